@@ -1009,7 +1009,7 @@ struct lri_ctx {
     if (op_quad) {
       quad_galerkin(U, true, rr);                      // U'AU, G'U, W(U)
       quad_init(V, m, rr, de->Snew, rr, 1, L);         // L = Z
-      quad_rows(false, rr, L, L2, Q, h, nsub);
+      quad_rows(false, rr, L, L2, h, nsub);
       HIPCHECK(hipMemcpyAsync(V, L, sizeof(double) * m * rr, hipMemcpyDeviceToDevice, stream));
     } else {
       de_galerkin(U, true, rr, de->Ga, de->gaT);       // U'AU, G'U
@@ -2439,9 +2439,9 @@ struct lri_ctx {
   // The stage arguments of the K (nside: operator A, D on K, forcing G) or L
   // sub-problem (operator B, no stencil, forcing H) with the Galerkin matrix M,
   // forcing projection hv and tensor T of the other side.
-  QuadStageArgs quad_stage_args(bool nside, int k, const double* M, const double* hv, const double* T, double h) {
+  QuadStepsArgs quad_steps_args(bool nside, int k, const double* M, const double* hv, const double* T, double h) {
     const int64_t rows_ = nside ? n : m;
-    QuadStageArgs Q;
+    QuadStepsArgs Q;
     Q.n = rows_;
     Q.k = k;
     Q.ld = rows_;
@@ -2463,35 +2463,58 @@ struct lri_ctx {
     }
     return Q;
   }
-  // N RK4 steps of the K (nside: M = V'BV, forcing G (H'V), tensor T, D on K) or
-  // L sub-problem (M = U'AU, forcing H (G'U), tensor W, no stencil) on X in place;
-  // scr holds 2 k columns, acc k columns (ld rows).  With `store`, the start of
-  // sub-step st is kept at store + st rows k.
-  void quad_rows_ex(bool nside, int k, const double* M, const double* hv, const double* T, double* X, double* scr,
-                    double* acc, double h, int64_t nsub, double* store) {
-    const int64_t rows_ = nside ? n : m;
-    QuadStageArgs Q = quad_stage_args(nside, k, M, hv, T, h);
-    Q.X0 = X;
-    Q.Acc = acc;
-    double* xa = scr;
-    double* xb = scr + rows_ * k;
-    const double* in[4] = {X, xa, xb, xa};
-    double* outp[4] = {xa, xb, xa, nullptr};
-    for (int64_t st = 0; st < nsub; ++st) {
-      if (store)
-        HIPCHECK(hipMemcpyAsync(store + st * rows_ * k, X, sizeof(double) * rows_ * k, hipMemcpyDeviceToDevice,
-                                stream));
-      for (int s = 0; s < 4; ++s) {
-        Q.stage = s;
-        Q.Xs = in[s];
-        Q.Xn = outp[s];
-        timed(LRI_KERNEL_DE, [&] { return launch_quad_stage(Q, stream); });
-      }
+  // N RK4 steps of the sub-problems A and (B.n > 0) B from quad_steps_args, in
+  // place on XA and XB; scrA and scrB hold k columns each.  With A.store (B.store),
+  // the start of sub-step st is kept at store + st rows k.  A launch takes two
+  // RK4 steps from one buffer to the other; an even number of launches ends where
+  // it began (for N = 1 the result is copied back).
+  void quad_steps(QuadStepsArgs A, double* XA, double* scrA, QuadStepsArgs B, double* XB, double* scrB,
+                  int64_t nsub) {
+    int64_t launches_left = (nsub + 1) / 2;
+    if (launches_left % 2 && nsub > 1) ++launches_left;
+    double *xa = XA, *ya = scrA, *xb = XB, *yb = scrB;
+    for (int64_t st = 0; st < nsub; --launches_left) {
+      A.nsteps = B.nsteps = nsub - st >= 2 && nsub - st > launches_left ? 2 : 1;
+      A.X = xa;
+      A.Xn = ya;
+      B.X = xb;
+      B.Xn = yb;
+      timed(LRI_KERNEL_DE, [&] { return launch_quad_steps(A, B, stream); });
+      std::swap(xa, ya);
+      std::swap(xb, yb);
+      st += A.nsteps;
+      if (A.store) A.store += A.nsteps * A.n * A.k;
+      if (B.store) B.store += B.nsteps * B.n * B.k;
+    }
+    if (xa != XA) {
+      HIPCHECK(hipMemcpyAsync(XA, xa, sizeof(double) * A.n * A.k, hipMemcpyDeviceToDevice, stream));
+      if (B.n) HIPCHECK(hipMemcpyAsync(XB, xb, sizeof(double) * B.n * B.k, hipMemcpyDeviceToDevice, stream));
     }
   }
-  void quad_rows(bool nside, int k, double* X, double* scr, double* acc, double h, int64_t nsub) {
-    quad_rows_ex(nside, k, nside ? de->Gb : de->Ga, nside ? de->hbT : de->gaT, nside ? quad_T : quad_W, X, scr, acc,
-                 h, nsub, nullptr);
+  // The K (nside: M = V'BV, forcing G (H'V), tensor T, D on K) or L sub-problem
+  // (M = U'AU, forcing H (G'U), tensor W, no stencil) with the Galerkin data of the DE
+  // work area, on X in place; scr holds k columns.
+  void quad_rows(bool nside, int k, double* X, double* scr, double h, int64_t nsub) {
+    quad_steps(quad_steps_args(nside, k, nside ? de->Gb : de->Ga, nside ? de->hbT : de->gaT, nside ? quad_T : quad_W, h),
+               X, scr, QuadStepsArgs{}, nullptr, nullptr, nsub);
+  }
+  // Both, from K = U S and L = V S' (the unconventional integrators: independent)
+  void quad_rows_pair(int k, double h, int64_t nsub) {
+    quad_init(U, n, k, S, (int)rcap, 0, K);
+    quad_init(V, m, k, S, (int)rcap, 1, L);
+    quad_steps(quad_steps_args(true, k, de->Gb, de->hbT, quad_T, h), K, K2,
+               quad_steps_args(false, k, de->Ga, de->gaT, quad_W, h), L, L2, nsub);
+  }
+  // The same for a reverse step, with the Galerkin data of qadj and the sub-step
+  // starts kept in stK and stL; work holds 2 max(n, m) k doubles.
+  void quad_rows_pair_kept(int k, double* work, double* stK, double* stL, double h, int64_t nsub) {
+    quad_init(U, n, k, S, (int)rcap, 0, K);
+    quad_init(V, m, k, S, (int)rcap, 1, L);
+    QuadStepsArgs A = quad_steps_args(true, k, qadj->Gb0, qadj->hbT0, qadj->T0, h);
+    QuadStepsArgs B = quad_steps_args(false, k, qadj->Ga0, qadj->gaT0, qadj->W0, h);
+    A.store = stK;
+    B.store = stL;
+    quad_steps(A, K, work, B, L, work + std::max(n, m) * k, nsub);
   }
   // Gram of X (rows x k) and the shifted first CholeskyQR factor
   void quad_gram(const double* X, int64_t rows_, int k, EpiArgs epi) {
@@ -2534,13 +2557,13 @@ struct lri_ctx {
     const EpiArgs none = de_epi();
     quad_galerkin(V, false, rr);  // V0'BV0, H'V0, T(V0)
     quad_init(U, n, rr, S, (int)rcap, 0, K);
-    quad_rows(true, rr, K, K2, P, h, nsub);
+    quad_rows(true, rr, K, K2, h, nsub);
     quad_gram(K, n, rr, shifted_chol(n));
     cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 0, 3);  // U1, R
     quad_galerkin(U, true, rr);                                    // U1'AU1, G'U1, W(U1)
     quad_sstep(rr, rr, small->Rtot, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
     quad_init(V, m, rr, de->Snew, rr, 1, L);
-    quad_rows(false, rr, L, L2, Q, h, nsub);
+    quad_rows(false, rr, L, L2, h, nsub);
     quad_gram(L, m, rr, shifted_chol(m));
     cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 2, 3);  // V1, S = R'
   }
@@ -2551,13 +2574,13 @@ struct lri_ctx {
     const EpiArgs none = de_epi();
     quad_galerkin(U, true, rr);  // U0'AU0, G'U0, W(U0)
     quad_init(V, m, rr, S, (int)rcap, 1, L);
-    quad_rows(false, rr, L, L2, Q, h, nsub);
+    quad_rows(false, rr, L, L2, h, nsub);
     quad_gram(L, m, rr, shifted_chol(m));
     cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 0, 3);  // V1, R
     quad_galerkin(V, false, rr);                                  // V1'BV1, H'V1, T(V1)
     quad_sstep(rr, rr, small->Rtot, rr, 1, de->Snew, rr, -1.0, h, nsub);  // S~ from R'
     quad_init(U, n, rr, de->Snew, rr, 0, K);
-    quad_rows(true, rr, K, K2, P, h, nsub);
+    quad_rows(true, rr, K, K2, h, nsub);
     quad_gram(K, n, rr, shifted_chol(n));
     cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 1, 3);  // U1, S = R
   }
@@ -2570,10 +2593,7 @@ struct lri_ctx {
       quad_galerkin(U, true, rr);
     }
     de_gal_fresh = false;
-    quad_init(U, n, rr, S, (int)rcap, 0, K);
-    quad_rows(true, rr, K, K2, P, h, nsub);
-    quad_init(V, m, rr, S, (int)rcap, 1, L);
-    quad_rows(false, rr, L, L2, Q, h, nsub);
+    quad_rows_pair(rr, h, nsub);
     quad_gram(K, n, rr, shifted_chol(n));
     cholqr_tail(K, K2, n, rr, U2, false, U, rr, de_epi(EPI_BUG_M), 0, 3);  // U1, M = U1'U0
     quad_gram(L, m, rr, shifted_chol(m));
@@ -2630,7 +2650,7 @@ struct lri_ctx {
   }
   // Reverse of the N RK4 steps of quad_rows_ex: store holds the sub-step starts,
   // ybar the cotangent of the result on entry and of the start on exit; the
-  // summed parameter cotangents go to sum.  work: 7 rows x k.
+  // summed parameter cotangents go to sum.  work: 6 rows x k.
   void quad_rows_reverse(bool nside, int k, const double* M, const double* hv, const double* T, const double* store,
                          double* ybar, double* work, double* part, double* sum, double h, int64_t nsub) {
     const int64_t rows_ = nside ? n : m;
@@ -2641,12 +2661,12 @@ struct lri_ctx {
     double* xa = x4 + sz;
     double* xb = xa + sz;
     double* ya = xb + sz;
-    double* accs = ya + sz;
     const int plen = quad_adj_part_len(k, op_q);
     const int grid = quad_adj_grid(rows_, k);
     HIPCHECK(hipMemsetAsync(part, 0, sizeof(double) * plen * grid, stream));
-    QuadStageArgs F = quad_stage_args(nside, k, M, hv, T, h);
-    F.Acc = accs;
+    QuadStepsArgs F = quad_steps_args(nside, k, M, hv, T, h);
+    F.nstages = 3;
+    F.stage_out = x2;  // x2, x3, x4
     QuadAdjStageArgs R;
     R.n = rows_;
     R.k = k;
@@ -2668,16 +2688,9 @@ struct lri_ctx {
     double* yb = ybar;
     double* yn = ya;
     for (int64_t st = nsub - 1; st >= 0; --st) {
-      double* y = const_cast<double*>(store) + st * sz;  // read-only for stages 0..2
-      F.X0 = y;
-      const double* fin[3] = {y, x2, x3};
-      double* fout[3] = {x2, x3, x4};
-      for (int s = 0; s < 3; ++s) {  // the stage inputs X2, X3, X4 of this sub-step
-        F.stage = s;
-        F.Xs = fin[s];
-        F.Xn = fout[s];
-        timed(LRI_KERNEL_DE, [&] { return launch_quad_stage(F, stream); });
-      }
+      const double* y = store + st * sz;
+      F.X = y;  // the stage inputs X2, X3, X4 of this sub-step
+      timed(LRI_KERNEL_DE, [&] { return launch_quad_steps(F, QuadStepsArgs{}, stream); });
       const double* in[4] = {y, x2, x3, x4};
       double* xbo = xa;
       const double* xbp = nullptr;
@@ -2749,10 +2762,7 @@ struct lri_ctx {
     }
     HIPCHECK(hipMemcpyAsync(qa->W0, quad_W, tsz, hipMemcpyDeviceToDevice, stream));
     HIPCHECK(hipMemcpyAsync(qa->T0, quad_T, tsz, hipMemcpyDeviceToDevice, stream));
-    quad_init(U, n, rr, S, (int)rcap, 0, K);
-    quad_rows_ex(true, rr, qa->Gb0, qa->hbT0, qa->T0, K, work, work + 2 * mx * rr, h, nsub, stK);
-    quad_init(V, m, rr, S, (int)rcap, 1, L);
-    quad_rows_ex(false, rr, qa->Ga0, qa->gaT0, qa->W0, L, work, work + 2 * mx * rr, h, nsub, stL);
+    quad_rows_pair_kept(rr, work, stK, stL, h, nsub);
     quad_gram(K, n, rr, shifted_chol(n));
     cholqr_tail(K, K2, n, rr, U2, false, U, rr, de_epi(EPI_BUG_M), 0, 3);  // U1, M = U1'U0
     HIPCHECK(hipMemcpyAsync(adj->RK, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
@@ -2930,7 +2940,9 @@ struct lri_ctx {
     if (op_q) HIPCHECK(hipMemcpyAsync(qa->hbT0, de->hbT, fsz, hipMemcpyDeviceToDevice, stream));
     HIPCHECK(hipMemcpyAsync(qa->T0, quad_T, tsz, hipMemcpyDeviceToDevice, stream));
     quad_init(U, n, rr, S, (int)rcap, 0, K);
-    quad_rows_ex(true, rr, qa->Gb0, qa->hbT0, qa->T0, K, work, work + 2 * mx * rr, h, nsub, stK);
+    QuadStepsArgs KA = quad_steps_args(true, rr, qa->Gb0, qa->hbT0, qa->T0, h);
+    KA.store = stK;
+    quad_steps(KA, K, work, QuadStepsArgs{}, nullptr, nullptr, nsub);
     quad_gram(K, n, rr, shifted_chol(n));
     cholqr_tail(K, K2, n, rr, U2, false, nullptr, 0, de_epi(), 0, 3);  // U1, R1
     HIPCHECK(hipMemcpyAsync(adj->RK, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
@@ -2941,7 +2953,9 @@ struct lri_ctx {
     HIPCHECK(hipMemcpyAsync(qa->W0, quad_W, tsz, hipMemcpyDeviceToDevice, stream));
     quad_sstep(rr, rr, adj->RK, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
     quad_init(V, m, rr, de->Snew, rr, 1, L);
-    quad_rows_ex(false, rr, qa->Ga0, qa->gaT0, qa->W0, L, work, work + 2 * mx * rr, h, nsub, stL);
+    QuadStepsArgs LA = quad_steps_args(false, rr, qa->Ga0, qa->gaT0, qa->W0, h);
+    LA.store = stL;
+    quad_steps(LA, L, work, QuadStepsArgs{}, nullptr, nullptr, nsub);
     quad_gram(L, m, rr, shifted_chol(m));
     cholqr_tail(L, L2, m, rr, V2, true, nullptr, 0, de_epi(), 0, 3);  // V1, R2
     HIPCHECK(hipMemcpyAsync(adj->RL, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
@@ -3102,10 +3116,7 @@ struct lri_ctx {
     const double h = dt / (double)nsub;
     quad_galerkin(V, false, rr);
     quad_galerkin(U, true, rr);
-    quad_init(U, n, rr, S, (int)rcap, 0, K);
-    quad_rows(true, rr, K, K2, P, h, nsub);
-    quad_init(V, m, rr, S, (int)rcap, 1, L);
-    quad_rows(false, rr, L, L2, Q, h, nsub);
+    quad_rows_pair(rr, h, nsub);
     HIPCHECK(hipMemcpyAsync(Uhat, U, sizeof(double) * n * rr, hipMemcpyDeviceToDevice, stream));
     EpiArgs eM;
     eM.kind = EPI_RA_M;
@@ -3171,10 +3182,7 @@ struct lri_ctx {
     }
     HIPCHECK(hipMemcpyAsync(qa->W0, quad_W, tsz, hipMemcpyDeviceToDevice, stream));
     HIPCHECK(hipMemcpyAsync(qa->T0, quad_T, tsz, hipMemcpyDeviceToDevice, stream));
-    quad_init(U, n, rr, S, (int)rcap, 0, K);
-    quad_rows_ex(true, rr, qa->Gb0, qa->hbT0, qa->T0, K, work, work + 2 * mx * rr, h, nsub, stK);
-    quad_init(V, m, rr, S, (int)rcap, 1, L);
-    quad_rows_ex(false, rr, qa->Ga0, qa->gaT0, qa->W0, L, work, work + 2 * mx * rr, h, nsub, stL);
+    quad_rows_pair_kept(rr, work, stK, stL, h, nsub);
     // the augmented bases, M, N, Sinit = M S0 N' and the completions' R factors
     for (int side = 0; side < 2; ++side) {
       const bool ns = side == 0;

@@ -413,18 +413,20 @@ struct TensorArgs {
 };
 hipError_t launch_tensor3(const TensorArgs& Q, double* out, hipStream_t st);
 
-// One RK4 stage (s = 0..3) of X' = A X + X M + g hv - N(X), N_ic = sum_ab (P X)_ia X_ib T_abc
-// (P = D when dd != nullptr, else I), over all n rows; X0 holds the state of the
-// RK4 step and is advanced in place by stage 3.
-struct QuadStageArgs {
+// `nsteps` RK4 steps (1 or 2) of X' = A X + X M + g hv - N(X), N_ic = sum_ab (P X)_ia X_ib T_abc
+// (P = D when dd != nullptr, else I), over all n rows, from X into Xn (another
+// buffer).  With `store`, the start of step s is kept at store + s n k.  With
+// `stage_out`, the inputs of stages 2, 3, 4 go to stage_out + (0, 1, 2) n k
+// (nstages = 3 then stops before the fourth stage; Xn may be nullptr).
+struct QuadStepsArgs {
   int64_t n = 0;
   int k = 0;
-  int64_t ld = 0;  // of X0, Xs, Xn, Acc
-  double* X0 = nullptr;
-  const double* Xs = nullptr;
+  int64_t ld = 0;  // of X and Xn
+  const double* X = nullptr;
   double* Xn = nullptr;
-  double* Acc = nullptr;
-  int stage = 0;
+  double* store = nullptr;
+  double* stage_out = nullptr;
+  int nsteps = 1, nstages = 4;
   double h = 0.0;
   const double* st_d = nullptr;  // A: symmetric tridiagonal (nullptr: none)
   const double* st_e = nullptr;
@@ -434,11 +436,14 @@ struct QuadStageArgs {
   int64_t ldg = 0;
   int q = 0;
   const double* hv = nullptr;    // q x k
-  const double* T = nullptr;     // k^3 (nullptr: no quadratic term)
+  const double* T = nullptr;     // k^3
   const double *dl = nullptr, *dd = nullptr, *du = nullptr;
   int dper = 0;
+  int blocks = 0;  // filled by the launcher
 };
-hipError_t launch_quad_stage(const QuadStageArgs& Q, hipStream_t st);
+constexpr int kQuadStepsLds = 19968;  // doubles: 156 KB of the 160 KB LDS
+// one launch for two independent sub-problems of the same k (B.n = 0: one)
+hipError_t launch_quad_steps(QuadStepsArgs A, QuadStepsArgs B, hipStream_t st);
 
 // N RK4 steps of S' = sgn (Ga S + S Gb + (gaT' hbT) - P(S)) (k x l), one workgroup.
 struct QuadSArgs {
@@ -462,7 +467,7 @@ struct QuadSArgs {
 hipError_t launch_quad_sstep(const QuadSArgs& Q, hipStream_t st);
 
 // Reverse (adjoint) of the quadratic sub-steps (see lri_quad_adj.hip).
-// One reverse RK4 stage s of X' = f(X) (f as in QuadStageArgs) over all rows:
+// One reverse RK4 stage s of X' = f(X) (f as in QuadStepsArgs) over all rows:
 // with Ybar the cotangent of the RK4 step's result and Xbp that of stage s + 1's
 // input, kbar = (h w_s / 6) Ybar + c_s h Xbp (w = 1, 2, 2, 1; c = 1/2, 1/2, 1),
 //   Xbo = J_f(X)' kbar,   Acc (=: s = 3 from Ybar, else +=) Xbo,

@@ -16,9 +16,9 @@
 //
 // with the third-order tensors T_abc = sum_j V_ja V_jb V_jc and
 // W_abc = sum_i (D U)_ia U_ib U_ic.  The sub-problems are no longer linear, so
-// every one of the N classical RK4 steps evaluates them: the K and L steps one
-// launch per RK4 stage over all rows (a stage needs the neighbouring rows of
-// the previous one), the S step in one workgroup.
+// every one of the N classical RK4 steps evaluates them: the K and L steps two
+// RK4 steps per launch over tiles of rows with a halo, the S step in one
+// workgroup.
 #include <algorithm>
 
 #include "lri_common.h"
@@ -115,108 +115,234 @@ hipError_t launch_tensor3(const TensorArgs& Q, double* out, hipStream_t st) {
 }
 
 // ----------------------------------------------------------------------------
-// One RK4 stage of the K or L sub-problem over all rows.  Workgroup: a tile of
-// 16 rows (4 waves).  The tile's rows (with one halo row on each side) are
-// staged in LDS, then
-//   f_ic = (A Xs)_ic + (Xs M)_ic + (g hv)_ic - N_ic,  N_ic = sum_ab (P Xs)_ia Xs_ib T_abc
-// (P = D when Q.dd, else the identity), and the RK4 bookkeeping of stage s:
-//   s < 3: Acc (=, +=) w_s f, Xn = X0 + c_s h f;   s = 3: X0 += h/6 (Acc + f).
-// The quadratic term is a product on the FP64 matrix cores,
-//   N (16 x k) = Z (16 x k^2) T (k^2 x k),  Z_i,(a + k b) = (P Xs)_ia Xs_ib,
-// T read once per tile in the k^2 order of its storage T[c + k (a + k b)]:
-// wave w takes column block w % nct (nct = ceil(k / 16)) and the w / nct-th of
-// the 4 / nct slices of the k^2 reduction; the slices are summed through LDS.
+// RK4 steps of the K or L sub-problem over a tile of rows, several stages per
+// launch.  A stage needs the neighbouring rows of the previous one only, so a
+// workgroup holds its kR - 2 kStepHalo rows with kStepHalo more on each side
+// and runs up to kStepHalo = 8 stages (two RK4 steps) without leaving the CU:
+// each stage makes one more row at either end stale, and after eight the
+// workgroup's own rows are still exact.  (One launch per stage was bound by its
+// launch latency: 9.4 us at n = 1000, k = 15, against about 0.7 us of FP64
+// work; eight stages of both sub-problems of the 1000 x 400 problem now take 19.7 us
+// in one launch, 2.5 us a stage: the solve went from 42.6 to 22.3 ms.)
+//
+//   f_ic = (A X)_ic + (X M)_ic + (g hv)_ic - N_ic,  N_ic = sum_ab (P X)_ia X_ib T_abc
+//
+// (P = D when Q.dd, else the identity).  X0, the RK4 accumulator and g hv of an
+// element stay in its thread's registers; the stage input X and P X are in LDS.
+// The quadratic term and X M are one product on the FP64 matrix cores,
+//   N - X M = sum_b diag(X_:b) (P X) T_:b:  +  X (-M),
+// a sum of k + 1 slabs (k x k each, in the k^2 order of the storage
+// T[c + k (a + k b)], the slab b = k holding -M).  A wave keeps its 16 rows of
+// P X in registers for the whole stage and scales them by X_:b, so a matrix
+// instruction costs one LDS read (of T) and one multiplication.  Wave w takes
+// rows 16 (w / 4) .. + 15, column block (w % 4) % nct (nct = ceil(k / 16)) and
+// every (4 / nct)-th slab; the slabs' sums meet in LDS in a fixed order.
 // ----------------------------------------------------------------------------
 
-constexpr int kStageRows = 16;
+constexpr int kStepHalo = 8;
 
-__global__ __launch_bounds__(256) void k_quad_stage(QuadStageArgs Q) {
-  __shared__ double xs[(kStageRows + 2) * kQuadMaxRank];  // rows r0 - 1 .. r0 + 16: xs[lr * k + c]
-  __shared__ double ps[kStageRows * kQuadMaxRank];        // (P Xs) rows r0 .. r0 + 15
-  __shared__ double nl[4][kStageRows * kQuadMaxRank];     // slices of N, [row * 32 + c]
-  const int k = Q.k, t = threadIdx.x;
+__host__ __device__ inline int quad_steps_pitch(int k) { return k | 1; }
+// doubles of LDS; t_lds: the tensor too
+__host__ __device__ inline int quad_steps_lds(int R, int k, bool t_lds) {
+  return (R + 2) * quad_steps_pitch(k) + R * quad_steps_pitch(k) + (R / 4) * 272 + 6 * R + k * k +
+         (t_lds ? k * k * k : 0);
+}
+
+// kQ = ceil(k / 4), kT: the tensor in LDS (else read from global memory)
+template <int kR, int kQ, bool kT>
+__global__ __launch_bounds__(16 * kR) void k_quad_steps(QuadStepsArgs Q0, QuadStepsArgs Q1) {
+  extern __shared__ double dyn[];
+  const QuadStepsArgs& Q = (int)blockIdx.x < Q0.blocks ? Q0 : Q1;
+  const int bid = (int)blockIdx.x - ((int)blockIdx.x < Q0.blocks ? 0 : Q0.blocks);
+  constexpr int kNT = 16 * kR, kNct = kQ > 4 ? 2 : 1, kNch = 4 / kNct, kE = kNct;  // kE elements per thread
+  constexpr int kOwn = kR - 2 * kStepHalo;
+  const int k = Q.k, kp = quad_steps_pitch(k), t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6, lr = lane & 15, lk = lane >> 4;
-  const int64_t r0 = (int64_t)blockIdx.x * kStageRows;
-  const int64_t n = Q.n;
-  // a row outside [0, n) takes its periodic image (used only by a periodic stencil)
-  for (int e = t; e < (kStageRows + 2) * k; e += blockDim.x) {
-    const int lrow = e % (kStageRows + 2), c = e / (kStageRows + 2);
-    int64_t ir = r0 + lrow - 1;
-    if (ir < 0) ir += n;
-    else if (ir >= n) ir -= n;
-    xs[lrow * k + c] = (ir >= 0 && ir < n) ? Q.Xs[ir + c * Q.ld] : 0.0;
-  }
-  __syncthreads();
-  for (int e = t; e < kStageRows * k; e += blockDim.x) {
-    const int lrow = e % kStageRows, c = e / kStageRows;
-    const int64_t i = r0 + lrow;
-    double p = 0.0;
-    if (i < n) {
-      const double xm = xs[lrow * k + c], x0 = xs[(lrow + 1) * k + c], xp = xs[(lrow + 2) * k + c];
-      const bool hasl = i > 0 || Q.dper, hasu = i < n - 1 || Q.dper;
-      p = Q.dd ? (Q.dd[i] * x0 + (hasl ? Q.dl[i] * xm : 0.0) + (hasu ? Q.du[i] * xp : 0.0)) : x0;
-    }
-    ps[lrow * k + c] = p;
-  }
-  __syncthreads();
-  const int nct = (k + 15) / 16, nch = 4 / nct;
-  if (Q.T) {
-    const int ct = wave % nct, ch = wave / nct;
-    const int kk2 = k * k;
-    const int clen = (kk2 + 4 * nch - 1) / (4 * nch) * 4;
-    const int kbeg = ch * clen, kend = min(kbeg + clen, kk2);
-    const int c = ct * 16 + lr;
-    f64x4_t acc = {0.0, 0.0, 0.0, 0.0};
-    // the tensor operand of the next k-step is loaded before this one's product
-    double bn = (kbeg + lk < kend && c < k) ? Q.T[c + (int64_t)k * (kbeg + lk)] : 0.0;
-    for (int kk0 = kbeg; kk0 < kend; kk0 += 4) {
-      const int kk = kk0 + lk;
-      const double b = bn;
-      bn = (kk + 4 < kend && c < k) ? Q.T[c + (int64_t)k * (kk + 4)] : 0.0;
-      const double a = kk < kend ? ps[lr * k + kk % k] * xs[(lr + 1) * k + kk / k] : 0.0;
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) nl[ch][(4 * u + lk) * kQuadMaxRank + c] = acc[u];
-  }
-  __syncthreads();
-  for (int e = t; e < kStageRows * k; e += blockDim.x) {
-    const int lrow = e % kStageRows, c = e / kStageRows;
-    const int64_t i = r0 + lrow;
-    if (i >= n) continue;
-    const double* xrow = xs + (lrow + 1) * k;
-    const double xm = xs[lrow * k + c], x0 = xrow[c], xp = xs[(lrow + 2) * k + c];
-    double f = 0.0;
-    // A Xs: symmetric tridiagonal, e[i] couples rows i and i + 1 (e[n-1]: n-1 and 0 when periodic)
+  const int n = (int)Q.n, r0 = bid * kOwn;
+  double* xs = dyn;                  // rows -1 .. kR of the tile: xs[(lrow + 1) * kp + c]
+  double* ps = xs + (kR + 2) * kp;   // P X
+  double* nl = ps + kR * kp;         // per wave 16 x 16 sums, pitch 17
+  double* cf = nl + (kR / 4) * 272;  // stencil coefficients: A lower, diagonal, upper, then P's
+  double* ms = cf + 6 * kR;          // -M (the slab b = k)
+  double* tl = ms + k * k;           // T
+  // row lrow of the tile is row (r0 - halo + lrow) mod n: the wrapped rows are the
+  // neighbours of a periodic stencil; without one their coupling is zero
+  for (int lrow = t; lrow < kR; lrow += kNT) {
+    int i = (r0 - kStepHalo + lrow) % n;
+    if (i < 0) i += n;
+    const bool first = i == 0, last = i == n - 1;
+    double al = 0.0, ad = 0.0, au = 0.0, pl = 0.0, pd = 1.0, pu = 0.0;
     if (Q.st_d) {
-      f = Q.st_d[i] * x0;
-      if (i > 0) f += Q.st_e[i - 1] * xm;
-      else if (Q.periodic) f += Q.st_e[n - 1] * xm;
-      if (i < n - 1) f += Q.st_e[i] * xp;
-      else if (Q.periodic) f += Q.st_e[n - 1] * xp;
+      ad = Q.st_d[i];
+      al = !first ? Q.st_e[i - 1] : Q.periodic ? Q.st_e[n - 1] : 0.0;
+      au = !last ? Q.st_e[i] : Q.periodic ? Q.st_e[n - 1] : 0.0;
     }
-    if (Q.M)
-      for (int l = 0; l < k; ++l) f += xrow[l] * Q.M[l + c * k];
-    for (int qq = 0; qq < Q.q; ++qq) f += Q.g[i + qq * Q.ldg] * Q.hv[qq + c * Q.q];
-    if (Q.T)
-      for (int ch = 0; ch < nch; ++ch) f -= nl[ch][lrow * kQuadMaxRank + c];
-    const int64_t o = i + c * Q.ld;
-    const int s = Q.stage;
-    if (s < 3) {
-      Q.Acc[o] = (s == 0 ? 0.0 : Q.Acc[o]) + stage_w(s) * f;
-      Q.Xn[o] = Q.X0[o] + stage_c(s) * Q.h * f;
-    } else {
-      Q.X0[o] = Q.X0[o] + (Q.h / 6.0) * (Q.Acc[o] + f);
+    if (Q.dd) {
+      pd = Q.dd[i];
+      pl = !first || Q.dper ? Q.dl[i] : 0.0;
+      pu = !last || Q.dper ? Q.du[i] : 0.0;
     }
+    cf[lrow] = al;
+    cf[kR + lrow] = ad;
+    cf[2 * kR + lrow] = au;
+    cf[3 * kR + lrow] = pl;
+    cf[4 * kR + lrow] = pd;
+    cf[5 * kR + lrow] = pu;
+  }
+  for (int e = t; e < k * k; e += kNT) ms[e] = Q.M ? -Q.M[(e / k) + (e % k) * k] : 0.0;  // ms[c + k a] = -M(a, c)
+  if (kT)
+    for (int e = t; e < k * k * k; e += kNT) tl[e] = Q.T[e];
+  for (int c = t; c < k; c += kNT) xs[c] = xs[(kR + 1) * kp + c] = 0.0;
+  // the thread's elements: row er, columns ec + 16 j
+  const int er = t % kR, ec = t / kR;
+  int gi = (r0 - kStepHalo + er) % n;
+  if (gi < 0) gi += n;
+  const bool own = er >= kStepHalo && er < kStepHalo + kOwn && r0 + er - kStepHalo < n;
+  double x0[kE], acc[kE], fg[kE];
+#pragma unroll
+  for (int j = 0; j < kE; ++j) {
+    const int c = ec + 16 * j;
+    x0[j] = acc[j] = fg[j] = 0.0;
+    if (c < k) {
+      x0[j] = Q.X[gi + c * Q.ld];
+      for (int qq = 0; qq < Q.q; ++qq) fg[j] += Q.g[gi + qq * Q.ldg] * Q.hv[qq + c * Q.q];
+      xs[(er + 1) * kp + c] = x0[j];
+    }
+  }
+  __syncthreads();
+  const double cal = cf[er], cad = cf[kR + er], cau = cf[2 * kR + er];
+  const double cpl = cf[3 * kR + er], cpd = cf[4 * kR + er], cpu = cf[5 * kR + er];
+  const int rt = (wave >> 2) * 16, ct = (wave & 3) % kNct, ch = (wave & 3) / kNct;
+  const int tc = min(ct * 16 + lr, k - 1);
+  const double h = Q.h;
+  for (int step = 0; step < Q.nsteps; ++step) {
+    if (Q.store && own) {
+#pragma unroll
+      for (int j = 0; j < kE; ++j)
+        if (ec + 16 * j < k) Q.store[step * Q.n * k + gi + (ec + 16 * j) * Q.n] = x0[j];
+    }
+    for (int s = 0; s < Q.nstages; ++s) {
+      double f[kE];
+#pragma unroll
+      for (int j = 0; j < kE; ++j) {
+        const int c = ec + 16 * j;
+        f[j] = 0.0;
+        if (c < k) {
+          const double xm = xs[er * kp + c], xc = xs[(er + 1) * kp + c], xp = xs[(er + 2) * kp + c];
+          ps[er * kp + c] = cpl * xm + cpd * xc + cpu * xp;
+          f[j] = cal * xm + cad * xc + cau * xp + fg[j];
+        }
+      }
+      __syncthreads();
+      {
+        double pr[kQ];
+        int to[kQ];
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+          const int a = 4 * j + lk;
+          to[j] = tc + k * min(a, k - 1);
+          pr[j] = a < k ? ps[(rt + lr) * kp + a] : 0.0;
+        }
+        const double* xr = xs + (rt + lr + 1) * kp;
+        f64x4_t a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
+        for (int b = ch; b < k; b += kNch) {
+          const double xb = xr[b];
+          const double* tb = (kT ? tl : Q.T) + k * k * b;
+          double bv[kQ];
+#pragma unroll
+          for (int j = 0; j < kQ; ++j) bv[j] = tb[to[j]];
+#pragma unroll
+          for (int j = 0; j < kQ; ++j) {
+            if (j & 1) a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(pr[j] * xb, bv[j], a1, 0, 0, 0);
+            else a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(pr[j] * xb, bv[j], a0, 0, 0, 0);
+          }
+        }
+        if (k % kNch == ch) {  // the slab b = k
+#pragma unroll
+          for (int j = 0; j < kQ; ++j) {
+            const double x = 4 * j + lk < k ? xr[min(4 * j + lk, k - 1)] : 0.0;
+            a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, ms[to[j]], a0, 0, 0, 0);
+          }
+        }
+        a0 += a1;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) nl[wave * 272 + (4 * u + lk) * 17 + lr] = a0[u];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kE; ++j) {
+        const int c = ec + 16 * j;
+        if (c < k) {
+          const double* nw = nl + ((er >> 4) * 4 + j) * 272 + (er & 15) * 17 + ec;
+#pragma unroll
+          for (int u = 0; u < kNch; ++u) f[j] -= nw[u * kNct * 272];
+          double x;
+          if (s < 3) {
+            acc[j] = (s == 0 ? 0.0 : acc[j]) + stage_w(s) * f[j];
+            x = x0[j] + stage_c(s) * h * f[j];
+            if (Q.stage_out && own) Q.stage_out[s * Q.n * k + gi + c * Q.n] = x;
+          } else {
+            x = x0[j] = x0[j] + (h / 6.0) * (acc[j] + f[j]);
+          }
+          xs[(er + 1) * kp + c] = x;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  if (Q.Xn && own) {
+#pragma unroll
+    for (int j = 0; j < kE; ++j)
+      if (ec + 16 * j < k) Q.Xn[gi + (ec + 16 * j) * Q.ld] = x0[j];
   }
 }
 
-hipError_t launch_quad_stage(const QuadStageArgs& Q, hipStream_t st) {
-  if (Q.k < 1 || Q.k > kQuadMaxRank || Q.n < 1 || Q.stage < 0 || Q.stage > 3 || Q.q < 0 || Q.q > kMaxForce)
-    return hipErrorInvalidValue;
-  const int64_t blocks = (Q.n + kStageRows - 1) / kStageRows;
-  hipLaunchKernelGGL(k_quad_stage, dim3((unsigned)blocks), dim3(256), 0, st, Q);
+namespace {
+
+template <int kR, int kQ>
+hipError_t run_quad_steps(const QuadStepsArgs& A, const QuadStepsArgs& B, unsigned grid, hipStream_t st) {
+  const int k = A.k;
+  const bool tl = quad_steps_lds(kR, k, true) <= kQuadStepsLds;
+  const size_t lds = sizeof(double) * quad_steps_lds(kR, k, tl);
+  if (tl) hipLaunchKernelGGL((k_quad_steps<kR, kQ, true>), dim3(grid), dim3(16 * kR), lds, st, A, B);
+  else hipLaunchKernelGGL((k_quad_steps<kR, kQ, false>), dim3(grid), dim3(16 * kR), lds, st, A, B);
   return hipGetLastError();
+}
+
+template <int kR>
+hipError_t dispatch_quad_steps(const QuadStepsArgs& A, const QuadStepsArgs& B, unsigned grid, hipStream_t st) {
+  switch ((A.k + 3) / 4) {
+    case 1: return run_quad_steps<kR, 1>(A, B, grid, st);
+    case 2: return run_quad_steps<kR, 2>(A, B, grid, st);
+    case 3: return run_quad_steps<kR, 3>(A, B, grid, st);
+    case 4: return run_quad_steps<kR, 4>(A, B, grid, st);
+    case 5: return run_quad_steps<kR, 5>(A, B, grid, st);
+    case 6: return run_quad_steps<kR, 6>(A, B, grid, st);
+    case 7: return run_quad_steps<kR, 7>(A, B, grid, st);
+    default: return run_quad_steps<kR, 8>(A, B, grid, st);
+  }
+}
+
+}  // namespace
+
+hipError_t launch_quad_steps(QuadStepsArgs A, QuadStepsArgs B, hipStream_t st) {
+  for (const QuadStepsArgs* Q : {&A, &B}) {
+    if (Q->n == 0 && Q == &B) continue;
+    if (Q->k < 1 || Q->k > kQuadMaxRank || Q->n < 1 || Q->n > (1 << 30) || Q->q < 0 || Q->q > kMaxForce || !Q->T ||
+        Q->nstages < 1 || Q->nstages > 4 || Q->nsteps < 1 || Q->nsteps * Q->nstages > kStepHalo ||
+        (Q->nsteps > 1 && Q->nstages != 4) || Q->X == Q->Xn)
+      return hipErrorInvalidValue;
+  }
+  if (B.n && B.k != A.k) return hipErrorInvalidValue;
+  // 32-row tiles (16 own rows) as long as all workgroups are resident at once;
+  // above that 64-row tiles, which repeat a third of their rows instead of half
+  auto blocks = [](int64_t rows, int own) { return (int)((rows + own - 1) / own); };
+  const bool small_tiles = blocks(A.n, 16) + blocks(B.n, 16) <= 512;
+  const int own = small_tiles ? 16 : 48;
+  A.blocks = blocks(A.n, own);
+  B.blocks = B.n ? blocks(B.n, own) : 0;
+  const unsigned grid = (unsigned)(A.blocks + B.blocks);
+  return small_tiles ? dispatch_quad_steps<32>(A, B, grid, st) : dispatch_quad_steps<64>(A, B, grid, st);
 }
 
 // ----------------------------------------------------------------------------
