@@ -284,7 +284,7 @@ struct lri_ctx {
   bool op_quad = false;
   double *op_dl = nullptr, *op_dd = nullptr, *op_du = nullptr;
   int op_dper = 0;
-  double *quad_part = nullptr, *quad_T = nullptr, *quad_W = nullptr, *quad_work = nullptr;
+  double *quad_part = nullptr, *quad_T = nullptr, *quad_W = nullptr;
   // matrix-ODE adjoint (allocated on first use): r x r data and the row work
   // (sub-step starts of K and L, stage inputs, cotangents, stage partials)
   QuadAdj* qadj = nullptr;
@@ -2527,11 +2527,10 @@ struct lri_ctx {
     A.epi = epi;
     rows(A);
   }
-  void quad_sstep(int k, int l, const double* S0, int lds0, int transS0, double* S1, int lds1, double sgn, double h,
+  void quad_sstep(int k, const double* S0, int lds0, int transS0, double* S1, int lds1, double sgn, double h,
                   int64_t nsub) {
     QuadSArgs Q;
     Q.k = k;
-    Q.l = l;
     Q.q = op_q;
     Q.S0 = S0;
     Q.lds0 = lds0;
@@ -2547,7 +2546,6 @@ struct lri_ctx {
     Q.sgn = sgn;
     Q.h = h;
     Q.nsub = nsub;
-    Q.work = quad_work;
     timed(LRI_KERNEL_SMALL, [&] { return launch_quad_sstep(Q, stream); });
   }
 
@@ -2561,7 +2559,7 @@ struct lri_ctx {
     quad_gram(K, n, rr, shifted_chol(n));
     cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 0, 3);  // U1, R
     quad_galerkin(U, true, rr);                                    // U1'AU1, G'U1, W(U1)
-    quad_sstep(rr, rr, small->Rtot, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
+    quad_sstep(rr, small->Rtot, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
     quad_init(V, m, rr, de->Snew, rr, 1, L);
     quad_rows(false, rr, L, L2, h, nsub);
     quad_gram(L, m, rr, shifted_chol(m));
@@ -2578,7 +2576,7 @@ struct lri_ctx {
     quad_gram(L, m, rr, shifted_chol(m));
     cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 0, 3);  // V1, R
     quad_galerkin(V, false, rr);                                  // V1'BV1, H'V1, T(V1)
-    quad_sstep(rr, rr, small->Rtot, rr, 1, de->Snew, rr, -1.0, h, nsub);  // S~ from R'
+    quad_sstep(rr, small->Rtot, rr, 1, de->Snew, rr, -1.0, h, nsub);  // S~ from R'
     quad_init(U, n, rr, de->Snew, rr, 0, K);
     quad_rows(true, rr, K, K2, h, nsub);
     quad_gram(K, n, rr, shifted_chol(n));
@@ -2603,7 +2601,7 @@ struct lri_ctx {
     cholqr_tail(L, L2, m, rr, V2, true, V, rr, eN, 0, 3);
     quad_galerkin(U2, true, rr);
     quad_galerkin(V2, false, rr);
-    quad_sstep(rr, rr, small->Sinit, rr, 0, S, (int)rcap, 1.0, h, nsub);
+    quad_sstep(rr, small->Sinit, rr, 0, S, (int)rcap, 1.0, h, nsub);
     std::swap(U, U2);
     std::swap(V, V2);
     de_gal_fresh = true;  // the Galerkin data and tensors now belong to U, V
@@ -2951,7 +2949,7 @@ struct lri_ctx {
     HIPCHECK(hipMemcpyAsync(qa->Ga0, de->Ga, rsz, hipMemcpyDeviceToDevice, stream));
     if (op_q) HIPCHECK(hipMemcpyAsync(qa->gaT0, de->gaT, fsz, hipMemcpyDeviceToDevice, stream));
     HIPCHECK(hipMemcpyAsync(qa->W0, quad_W, tsz, hipMemcpyDeviceToDevice, stream));
-    quad_sstep(rr, rr, adj->RK, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
+    quad_sstep(rr, adj->RK, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
     quad_init(V, m, rr, de->Snew, rr, 1, L);
     QuadStepsArgs LA = quad_steps_args(false, rr, qa->Ga0, qa->gaT0, qa->W0, h);
     LA.store = stL;
@@ -3129,7 +3127,7 @@ struct lri_ctx {
     complete_basis(L, V, m, rr, L2, L2 + m * rcap, Vhat + m * rr, eN);
     quad_galerkin(Uhat, true, k2);
     quad_galerkin(Vhat, false, k2);
-    quad_sstep(k2, k2, small->Sinit, k2, 0, small->Shat, k2, 1.0, h, nsub);
+    quad_sstep(k2, small->Sinit, k2, 0, small->Shat, k2, 1.0, h, nsub);
     ra_svd(k2, tol, rmax);
     return complete ? ra_rotate() : 0;
   }
@@ -3200,7 +3198,7 @@ struct lri_ctx {
     }
     quad_galerkin(Uhat, true, k2);   // Uhat'AUhat, G'Uhat, W(Uhat)
     quad_galerkin(Vhat, false, k2);  // Vhat'BVhat, H'Vhat, T(Vhat)
-    quad_sstep(k2, k2, small->Sinit, k2, 0, small->Shat, k2, 1.0, h, nsub);
+    quad_sstep(k2, small->Sinit, k2, 0, small->Shat, k2, 1.0, h, nsub);
     ra_svd(k2, tol, rmax);
     HIPCHECK(hipStreamSynchronize(stream));
     REQUIRE(*r_host == r1, "the cotangents' rank differs from the step's new rank (recomputed: " +
@@ -3737,7 +3735,7 @@ void free_ctx(lri_ctx* c) {
                   c->pkT_f32, c->pkN_hi, c->pkN_lo, c->pkT_hi,  c->pkT_lo,  c->partN,  c->partT,  c->gpart,
                   c->flags,  c->small,  c->svd_work, c->op_ad,  c->op_ae,   c->op_bd,   c->op_be,  c->op_G,
                   c->op_H,   c->de,     c->specQ[0], c->specLam[0], c->specF[0], c->op_dl, c->op_dd, c->op_du,
-                  c->quad_part, c->quad_T, c->quad_W, c->quad_work};
+                  c->quad_part, c->quad_T, c->quad_W};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   if (c->specF[1]) (void)hipFree(c->specF[1]);
@@ -4607,7 +4605,6 @@ int lri_set_operator_quadratic(lri_ctx* ctx, const double* dl, const double* dd,
     alloc(&ctx->quad_part, (size_t)((rows + 63) / 64) * k3);
     alloc(&ctx->quad_T, k3);
     alloc(&ctx->quad_W, k3);
-    alloc(&ctx->quad_work, 2 * k3);
     HIPCHECK(hipMemcpy(ctx->op_dl, dl, d * n, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(ctx->op_dd, dd, d * n, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(ctx->op_du, du, d * n, hipMemcpyHostToDevice));

@@ -445,24 +445,25 @@ constexpr int kQuadStepsLds = 19968;  // doubles: 156 KB of the 160 KB LDS
 // one launch for two independent sub-problems of the same k (B.n = 0: one)
 hipError_t launch_quad_steps(QuadStepsArgs A, QuadStepsArgs B, hipStream_t st);
 
-// N RK4 steps of S' = sgn (Ga S + S Gb + (gaT' hbT) - P(S)) (k x l), one workgroup.
+// N RK4 steps of S' = sgn (Ga S + S Gb + (gaT' hbT) - P(S)) (k x k), one workgroup.
+// With `store`, the input of stage s of step i is kept at store + (4 i + s) k^2.
 struct QuadSArgs {
-  int k = 0, l = 0, q = 0;
+  int k = 0, q = 0;
   const double* S0 = nullptr;
   int lds0 = 0;
   int transS0 = 0;
   double* S1 = nullptr;
   int lds1 = 0;
   const double* Ga = nullptr;   // k x k
-  const double* Gb = nullptr;   // l x l
+  const double* Gb = nullptr;   // k x k
   const double* gaT = nullptr;  // q x k
-  const double* hbT = nullptr;  // q x l
-  const double* W = nullptr;    // k^3, W[c + k (e + k f)] (nullptr: no quadratic term)
-  const double* T = nullptr;    // l^3
+  const double* hbT = nullptr;  // q x k
+  const double* W = nullptr;    // k^3, W[c + k (e + k f)]
+  const double* T = nullptr;    // k^3
   double sgn = 1.0;
   double h = 0.0;
   int64_t nsub = 0;
-  double* work = nullptr;       // k l k + l l k doubles
+  double* store = nullptr;
 };
 hipError_t launch_quad_sstep(const QuadSArgs& Q, hipStream_t st);
 

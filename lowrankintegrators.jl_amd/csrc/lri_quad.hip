@@ -347,109 +347,169 @@ hipError_t launch_quad_steps(QuadStepsArgs A, QuadStepsArgs B, hipStream_t st) {
 
 // ----------------------------------------------------------------------------
 // S sub-step: N RK4 steps of
-//   S' = sgn (Ga S + S Gb + cb - P(S)),  P_cd = sum_{a b} Z_abc T_abd,
-//   Z_abc = sum_e S_ea Y_ebc,  Y_ebc = sum_f S_fb W_efc,
-// S k x l in LDS, Y (k x l x k) and Z (l x l x k) in global scratch; one workgroup.
+//   S' = sgn (Ga S + S Gb + cb - P(S)),  P_cd = sum_ab Z_c,ab T_abd,  Z_c = S' W_c S,
+// S k x k, W_c = W(c, :, :), in one workgroup of 16 waves: the stages are a serial
+// chain, so what counts is the length of a stage.  Wave w takes c = w (and
+// c = w + 16 when k > 16): both products of Z_c stay in its registers, the result
+// layout of the FP64 matrix instruction (row 4 u + lane / 16, column lane % 16) being
+// the operand layout of the next one.  Z goes through LDS once, [a][c][b]; then
+// wave w takes a = w (and w + 16) of the contraction with T, and the waves' partial
+// sums of P (with slices of -(Ga S + S Gb)) meet in LDS in wave order.  For k <= 16
+// W, T, Ga and Gb are in registers for the whole launch, a stage is 12 to 14
+// matrix instructions a wave and three barriers: 1.3 us of the pipe's own time on
+// the one CU.  Measured with the products as separate passes over LDS (three
+// wave_gemm calls and scalar loops) 9.1 us a stage at k = 15; now 2.2 us (a
+// launch of 16 RK4 steps: 581 -> 142 us; at k = 24, 30 steps, the whole BUG solve 2.2 times
+// as fast together with the row kernel above).
+// For k > 16 the slices b < 16 and b >= 16 of Z take turns in LDS and W, T are read
+// from L2.
 // ----------------------------------------------------------------------------
 
-// kLds: the state, its RK4 work, the tensors W, T and the contractions Y, Z all
-// in LDS (quad_s_lds_doubles(k, l) <= kQuadSLds), else Y, Z in Q.work and W, T read
-// from global memory.
-constexpr int kQuadSLds = 20400;  // 159 KB of the 160 KB LDS
+constexpr int kSZPitch = 17;  // of Z's innermost index and of the partial sums: conflict-free both ways
 
-__host__ __device__ inline int quad_s_lds_doubles(int k, int l) {
-  return 5 * k * l + k * l * k + l * l * k + k * k * k + l * l * l;
-}
-
-template <bool kLds>
+template <int NB>  // 16-wide blocks: k <= 16 NB
 __global__ __launch_bounds__(1024) void k_quad_sstep(QuadSArgs Q) {
-  __shared__ double st_small[kLds ? 1 : 5 * kQuadMaxRank * kQuadMaxRank];
-  extern __shared__ double dyn[];
-  const int k = Q.k, l = Q.l, t = threadIdx.x, nt = blockDim.x;
-  const int kl = k * l;
-  double* base = kLds ? dyn : st_small;
-  double* y0 = base;
-  double* ys = y0 + kl;
-  double* acc = ys + kl;
-  double* cb = acc + kl;
-  double* pv = cb + kl;                          // the quadratic term P of a stage
-  double* Y = kLds ? pv + kl : Q.work;           // k x l x k: Y[c + k (e + k b)]
-  double* Z = Y + k * l * k;                     // l x l x k: Z[c + k (a + l b)]
-  const double* W = Q.W;
-  const double* T = Q.T;
-  if (kLds && Q.W) {
-    double* w = Z + l * l * k;
-    double* tt = w + k * k * k;
-    for (int e = t; e < k * k * k; e += nt) w[e] = Q.W[e];
-    for (int e = t; e < l * l * l; e += nt) tt[e] = Q.T[e];
-    W = w;
-    T = tt;
+  constexpr int NP = 16 * NB, NJ = 4 * NB;  // padded size, 4-deep reduction steps
+  __shared__ double sp[NP * (NP + 1)];             // S, zero-padded: sp[i * (NP + 1) + j]
+  __shared__ double zs[NP * NP * kSZPitch];        // Z: [(a * NP + c) * 17 + b]
+  __shared__ double pp_own[NB == 1 ? 16 * 16 * kSZPitch : 1];
+  // partial sums [wave][c][d]; for NB = 2 in zs, a 16-row block of c at a time
+  double* pp = NB == 1 ? pp_own : zs;
+  const int k = Q.k, t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 15, lk = lane >> 4;
+  constexpr int SP = NP + 1;
+  const bool elem = t < NP * NP;
+  const int ei = t / NP, ej = t % NP;
+  const bool live = elem && ei < k && ej < k;
+  double y0 = 0.0, cb = 0.0, acc = 0.0;
+  if (live) {
+    y0 = Q.transS0 ? Q.S0[ej + ei * Q.lds0] : Q.S0[ei + ej * Q.lds0];
+    for (int qq = 0; qq < Q.q; ++qq) cb += Q.gaT[qq + ei * Q.q] * Q.hbT[qq + ej * Q.q];
   }
-  for (int e = t; e < kl; e += nt) {
-    const int i = e % k, j = e / k;
-    y0[e] = Q.transS0 ? Q.S0[j + i * Q.lds0] : Q.S0[i + j * Q.lds0];
-    double s = 0.0;
-    for (int qq = 0; qq < Q.q; ++qq) s += Q.gaT[qq + i * Q.q] * Q.hbT[qq + j * Q.q];
-    cb[e] = s;
+  if (elem) sp[ei * SP + ej] = y0;
+  // W(c, e, f) and T(a, b, d), zero outside
+  auto wat = [&](int c, int e, int f) { return c < k && e < k && f < k ? Q.W[c + k * (e + k * f)] : 0.0; };
+  auto tat = [&](int a, int b, int d) { return a < k && b < k && d < k ? Q.T[d + k * (a + k * b)] : 0.0; };
+  double wr[NB == 1 ? 4 : 1], tr[NB == 1 ? 4 : 1];
+  if (NB == 1) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      wr[NB == 1 ? j : 0] = wat(wave, lr, 4 * j + lk);
+      tr[NB == 1 ? j : 0] = tat(wave, 4 * j + lk, lr);
+    }
+  }
+  // the linear part: reduction step jl of Ga S (waves 0 .. NJ - 1) or of S Gb (NJ .. 2 NJ - 1)
+  const int jl = wave % NJ, lin = wave < NJ ? 1 : wave < 2 * NJ ? 2 : 0;
+  double gl[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int i = 16 * b + lr, m = 4 * jl + lk;
+    gl[b] = lin && i < k && m < k ? -(lin == 1 ? Q.Ga[i + m * k] : Q.Gb[m + i * k]) : 0.0;
   }
   __syncthreads();
   const double h = Q.h;
-  for (int64_t step = 0; step < Q.nsub; ++step) {
-    for (int e = t; e < kl; e += nt) ys[e] = y0[e];
-    __syncthreads();
+  for (int64_t step = 0; step < Q.nsub; ++step)
     for (int s = 0; s < 4; ++s) {
-      if (Q.W) {
-        // on the matrix cores: Y_(c + k e), b = sum_f W_(c + k e), f S_fb;  Z_(c, a), b = sum_e Y_(c, e), b S_ea;
-        // P_ij = sum_(a + l b) Z_i, (a + l b) T_(a + l b), j  (into pv)
-        const int kk2 = k * k;
-        wave_gemm(kk2, l, k, 1, [&](int, int m, int f) { return W[m + kk2 * f]; },
-                  [&](int, int f, int b) { return ys[f + b * k]; },
-                  [&](int, int m, int b, double v) { Y[m + kk2 * b] = v; });
-        __syncthreads();
-        wave_gemm(k, l, k, l, [&](int b, int c, int e) { return Y[c + k * e + kk2 * b]; },
-                  [&](int, int e, int a) { return ys[e + a * k]; },
-                  [&](int b, int c, int a, double v) { Z[c + k * a + k * l * b] = v; });
-        __syncthreads();
-        wave_gemm(k, l, l * l, 1, [&](int, int i, int ab) { return Z[i + k * ab]; },
-                  [&](int, int ab, int j) { return T[j + l * ab]; },
-                  [&](int, int i, int j, double v) { pv[i + j * k] = v; });
-        __syncthreads();
-      }
-      double fv[(kQuadMaxRank * kQuadMaxRank + 1023) / 1024];
-      int cnt = 0;
-      for (int e = t; e < kl; e += nt, ++cnt) {
-        const int i = e % k, j = e / k;
-        double v = cb[e];
-        for (int m = 0; m < k; ++m) v += Q.Ga[i + m * k] * ys[m + j * k];
-        for (int m = 0; m < l; ++m) v += ys[i + m * k] * Q.Gb[m + j * l];
-        if (Q.W) v -= pv[e];
-        fv[cnt] = Q.sgn * v;
-      }
-      __syncthreads();  // every stage input read before it is replaced
-      cnt = 0;
-      for (int e = t; e < kl; e += nt, ++cnt) {
-        const double f = fv[cnt];
-        if (s < 3) {
-          acc[e] = (s == 0 ? 0.0 : acc[e]) + stage_w(s) * f;
-          ys[e] = y0[e] + stage_c(s) * h * f;
-        } else {
-          y0[e] = y0[e] + (h / 6.0) * (acc[e] + f);
+      if (Q.store && live) Q.store[(step * 4 + s) * k * k + ei + ej * k] = sp[ei * SP + ej];
+      f64x4_t pa[NB][NB];
+#pragma unroll
+      for (int cbk = 0; cbk < NB; ++cbk)
+#pragma unroll
+        for (int db = 0; db < NB; ++db) pa[cbk][db] = (f64x4_t){0.0, 0.0, 0.0, 0.0};
+      for (int bb = 0; bb < NB; ++bb) {  // columns b of Z
+        double sb[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) sb[j] = sp[(4 * j + lk) * SP + 16 * bb + lr];
+        for (int c = wave; c < k; c += 16) {
+          f64x4_t yc[NB];
+#pragma unroll
+          for (int eb = 0; eb < NB; ++eb) {  // Y = W_c S, rows 16 eb ..
+            f64x4_t a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+              const double w = NB == 1 ? wr[NB == 1 ? j : 0] : wat(c, 16 * eb + lr, 4 * j + lk);
+              if (j & 1) a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(w, sb[j], a1, 0, 0, 0);
+              else a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(w, sb[j], a0, 0, 0, 0);
+            }
+            yc[eb] = a0 + a1;
+          }
+#pragma unroll
+          for (int ab = 0; ab < NB; ++ab) {  // Z_c = S' Y, rows 16 ab ..
+            f64x4_t a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+              const double sa = ab == bb ? sb[j] : sp[(4 * j + lk) * SP + 16 * ab + lr];
+              if (j & 1) a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(sa, yc[j / 4][j % 4], a1, 0, 0, 0);
+              else a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(sa, yc[j / 4][j % 4], a0, 0, 0, 0);
+            }
+            a0 += a1;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) zs[((16 * ab + 4 * u + lk) * NP + c) * kSZPitch + lr] = a0[u];
+          }
         }
+        if (bb == 0 && lin) {
+#pragma unroll
+          for (int cbk = 0; cbk < NB; ++cbk)
+#pragma unroll
+            for (int db = 0; db < NB; ++db) {
+              const double sv = lin == 1 ? sp[(4 * jl + lk) * SP + 16 * db + lr] : sp[(16 * cbk + lr) * SP + 4 * jl + lk];
+              pa[cbk][db] = lin == 1 ? __builtin_amdgcn_mfma_f64_16x16x4f64(gl[cbk], sv, pa[cbk][db], 0, 0, 0)
+                                     : __builtin_amdgcn_mfma_f64_16x16x4f64(sv, gl[db], pa[cbk][db], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+        for (int a = wave; a < k; a += 16) {
+#pragma unroll
+          for (int db = 0; db < NB; ++db)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const double tv = NB == 1 ? tr[NB == 1 ? j : 0] : tat(a, 16 * bb + 4 * j + lk, 16 * db + lr);
+#pragma unroll
+              for (int cbk = 0; cbk < NB; ++cbk) {
+                const int c = 16 * cbk + lr;
+                // the rows c >= k of zs are never written
+                const double z = c < k ? zs[(a * NP + c) * kSZPitch + 4 * j + lk] : 0.0;
+                pa[cbk][db] = __builtin_amdgcn_mfma_f64_16x16x4f64(z, tv, pa[cbk][db], 0, 0, 0);
+              }
+            }
+        }
+        if (NB > 1) __syncthreads();  // zs is free again
+      }
+      double p = 0.0;
+#pragma unroll
+      for (int cbk = 0; cbk < NB; ++cbk) {
+#pragma unroll
+        for (int db = 0; db < NB; ++db)
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            pp[((wave * 16 + 4 * u + lk) * NB + db) * kSZPitch + lr] = pa[cbk][db][u];
+        __syncthreads();
+        if (elem && (ei >> 4) == cbk) {
+#pragma unroll
+          for (int w = 0; w < 16; ++w) p += pp[((w * 16 + (ei & 15)) * NB + (ej >> 4)) * kSZPitch + (ej & 15)];
+        }
+        if (NB > 1) __syncthreads();
+      }
+      if (live) {
+        const double f = Q.sgn * (cb - p);
+        double x;
+        if (s < 3) {
+          acc = (s == 0 ? 0.0 : acc) + stage_w(s) * f;
+          x = y0 + stage_c(s) * h * f;
+        } else {
+          x = y0 = y0 + (h / 6.0) * (acc + f);
+        }
+        sp[ei * SP + ej] = x;
       }
       __syncthreads();
     }
-  }
-  for (int e = t; e < kl; e += nt) Q.S1[(e % k) + (e / k) * Q.lds1] = y0[e];
+  if (Q.S1 && live) Q.S1[ei + ej * Q.lds1] = y0;
 }
 
 hipError_t launch_quad_sstep(const QuadSArgs& Q, hipStream_t st) {
-  if (Q.k < 1 || Q.l < 1 || Q.k > kQuadMaxRank || Q.l > kQuadMaxRank || Q.q < 0 || Q.q > kMaxForce || !Q.work)
+  if (Q.k < 1 || Q.k > kQuadMaxRank || Q.q < 0 || Q.q > kMaxForce || !Q.W || !Q.T || !Q.Ga || !Q.Gb)
     return hipErrorInvalidValue;
-  const int need = quad_s_lds_doubles(Q.k, Q.l);
-  if (need <= kQuadSLds)
-    hipLaunchKernelGGL(k_quad_sstep<true>, dim3(1), dim3(1024), sizeof(double) * need, st, Q);
-  else
-    hipLaunchKernelGGL(k_quad_sstep<false>, dim3(1), dim3(1024), 0, st, Q);
+  if (Q.k <= 16) hipLaunchKernelGGL(k_quad_sstep<1>, dim3(1), dim3(1024), 0, st, Q);
+  else hipLaunchKernelGGL(k_quad_sstep<2>, dim3(1), dim3(1024), 0, st, Q);
   return hipGetLastError();
 }
 
