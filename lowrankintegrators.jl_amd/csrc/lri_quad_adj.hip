@@ -289,16 +289,16 @@ hipError_t launch_part_sum(const double* part, int count, int len, double* out, 
 }
 
 // ----------------------------------------------------------------------------
-// Reverse of the S sub-step, one workgroup of 1024 threads (16 waves).  The
-// k x l matrices live in LDS; the third-order intermediates in three buffers
-// B0, B1, B2 (LDS when they and T fit, else Q.work), reused as they die:
-//   forward f:  Y_ebc = sum_f X_fb W_efc -> B0,  Z_abc = sum_e X_ea Y_ebc -> B1,
-//               P = Z' T (k x l);
-//   reverse:    Y -> B0, Z -> B1;  Tbar_abj -= sum_i Z_abi pb_ij, X1_ebj = sum_a X_ea T_abj -> B0;
-//               Zt_efj = sum_b X_fb X1_ebj -> B1;  Wbar_efi -= sum_j pb_ij Zt_efj,
-//               C_efj = sum_i pb_ij W_efi -> B0;  D1_ebj = sum_f C_efj X_fb -> B1,
-//               E1_faj = sum_e C_efj X_ea -> B2;
-//               J_P' pb = sum_bj D1_ibj T_abj + sum_a'j E1_ia'j T_a'aj,
+// Reverse of the S sub-step for k > 16, one workgroup of 1024 threads (16 waves).
+// k_quad_sstep has left the stage inputs X in Q.work.  The k x l matrices live in
+// LDS; the third-order intermediates in three buffers B0, B1, B2 (LDS when they
+// and T fit, else Q.work), reused as they die:
+//   Y_ebc = sum_f X_fb W_efc -> B0,  Z_abc = sum_e X_ea Y_ebc -> B1;
+//   Tbar_abj -= sum_i Z_abi pb_ij, X1_ebj = sum_a X_ea T_abj -> B0;
+//   Zt_efj = sum_b X_fb X1_ebj -> B1;  Wbar_efi -= sum_j pb_ij Zt_efj,
+//   C_efj = sum_i pb_ij W_efi -> B0;  D1_ebj = sum_f C_efj X_fb -> B1,
+//   E1_faj = sum_e C_efj X_ea -> B2;
+//   J_P' pb = sum_bj D1_ibj T_abj + sum_a'j E1_ia'j T_a'aj,
 // every contraction a product on the FP64 matrix cores (wave_gemm).
 // ----------------------------------------------------------------------------
 
@@ -308,39 +308,6 @@ struct SAdjBufs {
   double *B0, *B1, *B2;
   const double* T;  // the tensor T (LDS copy or Q.T)
 };
-
-// out = f(X) (k x l, ld k); tmp: k x l scratch
-__device__ void sadj_f(const QuadSAdjArgs& Q, const double* X, double* out, const double* cb, double* tmp,
-                       const SAdjBufs& w) {
-  const int k = Q.k, l = Q.l, t = threadIdx.x, nt = blockDim.x;
-  const double* W = Q.W;
-  const double* T = w.T;
-  double* B0 = w.B0;
-  double* B1 = w.B1;
-  if (W) {
-    wave_gemm(k * k, l, k, 1, [&](int, int m, int kk) { return W[m + k * k * kk]; },
-              [&](int, int kk, int nn) { return X[kk + nn * k]; },
-              [&](int, int m, int nn, double v) { B0[m + k * k * nn] = v; });
-    __syncthreads();
-    wave_gemm(k, l, k, l, [&](int b, int c, int e) { return B0[c + k * e + k * k * b]; },
-              [&](int, int e, int a) { return X[e + a * k]; },
-              [&](int b, int c, int a, double v) { B1[c + k * a + k * l * b] = v; });
-    __syncthreads();
-    wave_gemm(k, l, l * l, 1, [&](int, int i, int ab) { return B1[i + k * ab]; },
-              [&](int, int ab, int j) { return T[j + l * ab]; },
-              [&](int, int i, int j, double v) { tmp[i + j * k] = v; });
-    __syncthreads();
-  }
-  for (int e = t; e < k * l; e += nt) {
-    const int i = e % k, j = e / k;
-    double v = cb[e];
-    for (int m = 0; m < k; ++m) v += Q.Ga[i + m * k] * X[m + j * k];
-    for (int m = 0; m < l; ++m) v += X[i + m * k] * Q.Gb[m + j * l];
-    if (W) v -= tmp[e];
-    out[e] = Q.sgn * v;
-  }
-  __syncthreads();
-}
 
 // xb = J_f(X)' kb; accumulates Gab, Gbb, cbar (LDS) and Wb, Tb (global)
 __device__ void sadj_rev(const QuadSAdjArgs& Q, const double* X, const double* kb, double* pb, double* xb,
@@ -424,9 +391,9 @@ __device__ void sadj_rev(const QuadSAdjArgs& Q, const double* X, const double* k
 
 }  // namespace
 
-// LDS doubles: 11 k l + k^2 + l^2 for the matrices, then (when they fit) the
+// LDS doubles: 8 k l + k^2 + l^2 for the matrices, then (when they fit) the
 // three intermediate buffers and T
-__host__ __device__ inline int quad_sadj_small_doubles(int k, int l) { return 11 * k * l + k * k + l * l; }
+__host__ __device__ inline int quad_sadj_small_doubles(int k, int l) { return 8 * k * l + k * k + l * l; }
 __host__ __device__ inline int quad_sadj_r3(int k, int l) { return k * l * (k > l ? k : l); }
 constexpr int kSAdjLdsMax = 20480;  // 160 KB
 
@@ -434,16 +401,13 @@ template <bool kLds>
 __global__ __launch_bounds__(1024) void k_quad_sadj(QuadSAdjArgs Q) {
   extern __shared__ double lds[];
   const int k = Q.k, l = Q.l, kl = k * l, t = threadIdx.x, nt = blockDim.x;
-  double* y = lds;
-  double* fv = y + kl;
-  double* x = fv + kl;
+  double* x = lds;
   double* kb = x + kl;
   double* pb = kb + kl;
   double* xb = pb + kl;
   double* yb = xb + kl;
   double* acc = yb + kl;
-  double* cb = acc + kl;
-  double* cbar = cb + kl;
+  double* cbar = acc + kl;
   double* tmp = cbar + kl;
   double* Gab = tmp + kl;
   double* Gbb = Gab + k * k;
@@ -467,11 +431,7 @@ __global__ __launch_bounds__(1024) void k_quad_sadj(QuadSAdjArgs Q) {
   const double h = Q.h;
   for (int e = t; e < kl; e += nt) {
     const int i = e % k, j = e / k;
-    y[e] = Q.S0[i + j * Q.lds0];
     yb[e] = Q.Sb1[i + j * Q.ldsb1];
-    double s = 0.0;
-    for (int qq = 0; qq < Q.q; ++qq) s += Q.gaT[qq + i * Q.q] * Q.hbT[qq + j * Q.q];
-    cb[e] = s;
     cbar[e] = 0.0;
   }
   for (int e = t; e < k * k; e += nt) Gab[e] = 0.0;
@@ -481,28 +441,6 @@ __global__ __launch_bounds__(1024) void k_quad_sadj(QuadSAdjArgs Q) {
     for (int e = t; e < l * l * l; e += nt) Q.Tb[e] = 0.0;
   }
   __syncthreads();
-  // forward trajectory, keeping every stage input
-  for (int64_t st = 0; st < Q.nsub; ++st) {
-    double* X4 = store + st * 4 * kl;
-    for (int e = t; e < kl; e += nt) {
-      X4[e] = y[e];
-      x[e] = y[e];
-    }
-    __syncthreads();
-    for (int s = 0; s < 4; ++s) {
-      sadj_f(Q, x, fv, cb, tmp, w);
-      for (int e = t; e < kl; e += nt) {
-        if (s < 3) {
-          acc[e] = (s == 0 ? 0.0 : acc[e]) + stage_w(s) * fv[e];
-          x[e] = y[e] + stage_c(s) * h * fv[e];
-          X4[(s + 1) * kl + e] = x[e];
-        } else {
-          y[e] = y[e] + (h / 6.0) * (acc[e] + fv[e]);
-        }
-      }
-      __syncthreads();
-    }
-  }
   // reverse
   for (int64_t st = Q.nsub - 1; st >= 0; --st) {
     const double* X4 = store + st * 4 * kl;
@@ -536,11 +474,176 @@ __global__ __launch_bounds__(1024) void k_quad_sadj(QuadSAdjArgs Q) {
   }
 }
 
+// ----------------------------------------------------------------------------
+// The same for k <= 16 in registers, as k_quad_sstep.  With P_cd = sum_ab Z_c,ab T_abd,
+// Z_c = S' W_c S, and pb the cotangent of sgn P, wave w takes c = w and a = w:
+//   Zb^a_cb = sum_d pb_cd T_abd,   Tbar^a_bd -= sum_c Z_c,ab pb_cd,
+//   Sbar' -= Zb_c (W_c S)' + Zb_c' (W_c' S)',   Wbar_c -= S Zb_c S'
+// (Sbar' = its transpose).  Z and Zb cross between the two roles through LDS; W_c, W_c',
+// T_a, the sums Tbar^a and Wbar_c, and those of Ga and Gb (waves 8 and 9) stay in
+// registers over all stages.  40 matrix instructions a wave and stage: 4.3 us of
+// the one CU's pipe.  The general kernel took about 60 us a reverse stage at k = 16
+// (1927 us a launch of 7 RK4 steps, its forward stages included), this one 6.8 us
+// (191 us, and 67 us for k_quad_sstep).
+// ----------------------------------------------------------------------------
+
+__global__ __launch_bounds__(1024) void k_quad_sadj16(QuadSAdjArgs Q) {
+  constexpr int SP = 17;
+  __shared__ double sp[16 * SP];       // the stage input X
+  __shared__ double pbp[16 * SP];      // sgn kbar
+  __shared__ double zs[256 * SP];      // Z: [(a * 16 + c) * 17 + b]
+  __shared__ double zb[256 * SP];      // Zb: [(c * 16 + a) * 17 + b]
+  __shared__ double pp[256 * SP];      // partial Sbar': [(wave * 16 + a) * 17 + e]
+  const int k = Q.k, k2 = k * k, t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 15, lk = lane >> 4;
+  const int ei = (t >> 4) & 15, ej = t & 15;
+  const bool elem = t < 256, live = elem && ei < k && ej < k;
+  const double* store = Q.work;  // [sub-step][stage][k k]: the stage inputs
+  const double h = Q.h;
+  double wr[4], wt[4], td[4], gl[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = 4 * j + lk;
+    const bool in = wave < k && lr < k && i < k;
+    wr[j] = in ? Q.W[wave + k * (lr + k * i)] : 0.0;
+    wt[j] = in ? Q.W[wave + k * (i + k * lr)] : 0.0;
+    td[j] = in ? Q.T[i + k * (wave + k * lr)] : 0.0;
+    // the linear part, reduction step j = wave % 4: Ga (waves 0 - 3), Gb (waves 4 - 7)
+    gl[j] = 0.0;
+    if (lr < k && i < k && wave < 8 && j == (wave & 3)) gl[j] = wave < 4 ? -Q.Ga[i + lr * k] : -Q.Gb[lr + i * k];
+  }
+  const double glw = gl[0] + gl[1] + gl[2] + gl[3];  // the one that is set
+  const int jl = wave & 3;
+  f64x4_t accT = {0.0, 0.0, 0.0, 0.0}, accW = accT, accG = accT;
+  double yb = 0.0, xb = 0.0, acc = 0.0, cbar = 0.0;
+  if (live) yb = Q.Sb1[ei + ej * Q.ldsb1];
+  double xn = live ? store[(Q.nsub * 4 - 1) * k2 + ei + ej * k] : 0.0;
+  for (int64_t q = Q.nsub * 4 - 1; q >= 0; --q) {
+    const int s = (int)(q & 3);
+    if (elem) {
+      const double pb = Q.sgn * ((h * stage_w(s) / 6.0) * yb + (s < 3 ? stage_c(s) * h * xb : 0.0));
+      sp[ei * SP + ej] = xn;
+      pbp[ei * SP + ej] = pb;
+      cbar += pb;
+      if (live && q > 0) xn = store[(q - 1) * k2 + ei + ej * k];
+    }
+    __syncthreads();
+    double sb[4], sa[4], pa[4], pt[4];  // X and pb as operands: [i][lr] and [lr][i], i = 4 j + lk
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = 4 * j + lk;
+      sb[j] = sp[i * SP + lr];
+      sa[j] = sp[lr * SP + i];
+      pa[j] = pbp[lr * SP + i];
+      pt[j] = pbp[i * SP + lr];
+    }
+    f64x4_t y = {0.0, 0.0, 0.0, 0.0}, yt = y, ytt = y, z = y, za = y;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      y = __builtin_amdgcn_mfma_f64_16x16x4f64(wr[j], sb[j], y, 0, 0, 0);      // W_c S
+      za = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[j], td[j], za, 0, 0, 0);    // Zb^a
+      yt = __builtin_amdgcn_mfma_f64_16x16x4f64(sb[j], wr[j], yt, 0, 0, 0);    // (W_c S)'
+      ytt = __builtin_amdgcn_mfma_f64_16x16x4f64(sb[j], wt[j], ytt, 0, 0, 0);  // (W_c' S)'
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z = __builtin_amdgcn_mfma_f64_16x16x4f64(sb[j], y[j], z, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      zs[((4 * u + lk) * 16 + wave) * SP + lr] = z[u];
+      zb[((4 * u + lk) * 16 + wave) * SP + lr] = za[u];
+    }
+    __syncthreads();
+    f64x4_t ps = {0.0, 0.0, 0.0, 0.0}, ps2 = ps, hh = ps;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = 4 * j + lk;
+      const double zbj = zb[(wave * 16 + lr) * SP + i];                  // Zb_c [a = lr][b = i]
+      ps = __builtin_amdgcn_mfma_f64_16x16x4f64(zbj, yt[j], ps, 0, 0, 0);
+      hh = __builtin_amdgcn_mfma_f64_16x16x4f64(zbj, sa[j], hh, 0, 0, 0);  // Zb_c S'
+      const double zbt = zb[(wave * 16 + i) * SP + lr];                  // Zb_c'
+      ps2 = __builtin_amdgcn_mfma_f64_16x16x4f64(zbt, ytt[j], ps2, 0, 0, 0);
+      const double zj = zs[(wave * 16 + i) * SP + lr];                   // Z^a [c = i][b = lr]
+      accT = __builtin_amdgcn_mfma_f64_16x16x4f64(zj, pt[j], accT, 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) accW = __builtin_amdgcn_mfma_f64_16x16x4f64(sa[j], hh[j], accW, 0, 0, 0);
+    if (wave < 8) {  // - (Ga' pb)' and - (pb Gb')'
+      const double o = pbp[(wave < 4 ? (4 * jl + lk) * SP + lr : lr * SP + 4 * jl + lk)];
+      ps = wave < 4 ? __builtin_amdgcn_mfma_f64_16x16x4f64(o, glw, ps, 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f64_16x16x4f64(glw, o, ps, 0, 0, 0);
+    } else if (wave == 8) {  // Gab += pb X'
+#pragma unroll
+      for (int j = 0; j < 4; ++j) accG = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[j], sa[j], accG, 0, 0, 0);
+    } else if (wave == 9) {  // Gbb += X' pb
+#pragma unroll
+      for (int j = 0; j < 4; ++j) accG = __builtin_amdgcn_mfma_f64_16x16x4f64(sb[j], pt[j], accG, 0, 0, 0);
+    }
+    ps += ps2;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) pp[(wave * 16 + 4 * u + lk) * SP + lr] = ps[u];
+    __syncthreads();
+    if (elem) {
+      double v = 0.0;
+#pragma unroll
+      for (int w = 0; w < 16; ++w) v += pp[(w * 16 + ej) * SP + ei];
+      xb = live ? -v : 0.0;
+      acc = (s == 3 ? yb : acc) + xb;
+      if (s == 0) yb = acc;
+    }
+  }
+  if (live) Q.Sb0[ei + ej * k] = yb;
+  __syncthreads();
+  if (elem) sp[ei * SP + ej] = cbar;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int i = 4 * u + lk;
+    if (i < k && lr < k) {
+      if (wave < k) {
+        Q.Tb[lr + k * (wave + k * i)] = -accT[u];
+        Q.Wb[wave + k * (i + k * lr)] = -accW[u];
+      }
+      if (wave == 8) Q.Gab[i + lr * k] = accG[u];
+      if (wave == 9) Q.Gbb[i + lr * k] = accG[u];
+    }
+  }
+  __syncthreads();
+  for (int e = t; e < Q.q * k; e += blockDim.x) {  // cb_ij = sum_q gaT_qi hbT_qj
+    const int qq = e % Q.q, i = e / Q.q;
+    double va = 0.0, vb = 0.0;
+    for (int j = 0; j < k; ++j) {
+      va += Q.hbT[qq + j * Q.q] * sp[i * SP + j];
+      vb += Q.gaT[qq + j * Q.q] * sp[j * SP + i];
+    }
+    Q.gaTb[e] = va;
+    Q.hbTb[e] = vb;
+  }
+}
+
 hipError_t launch_quad_sadj(const QuadSAdjArgs& Q, hipStream_t st) {
   if (Q.k < 1 || Q.l < 1 || Q.k > kQuadMaxRank || Q.l > kQuadMaxRank || Q.q < 0 || Q.q > kMaxForce || !Q.work ||
       Q.nsub < 1 || !Q.S0 || !Q.Sb1 || !Q.Sb0 || !Q.Ga || !Q.Gb || !Q.Gab || !Q.Gbb ||
-      (Q.q > 0 && (!Q.gaT || !Q.hbT || !Q.gaTb || !Q.hbTb)) || (Q.W && (!Q.T || !Q.Wb || !Q.Tb)))
+      (Q.q > 0 && (!Q.gaT || !Q.hbT || !Q.gaTb || !Q.hbTb)) || Q.k != Q.l || !Q.W || !Q.T || !Q.Wb || !Q.Tb)
     return hipErrorInvalidValue;
+  QuadSArgs F;  // the stage inputs
+  F.k = Q.k;
+  F.q = Q.q;
+  F.S0 = Q.S0;
+  F.lds0 = Q.lds0;
+  F.Ga = Q.Ga;
+  F.Gb = Q.Gb;
+  F.gaT = Q.gaT;
+  F.hbT = Q.hbT;
+  F.W = Q.W;
+  F.T = Q.T;
+  F.sgn = Q.sgn;
+  F.h = Q.h;
+  F.nsub = Q.nsub;
+  F.store = Q.work;
+  const hipError_t e = launch_quad_sstep(F, st);
+  if (e != hipSuccess) return e;
+  if (Q.k <= 16) {
+    hipLaunchKernelGGL(k_quad_sadj16, dim3(1), dim3(1024), 0, st, Q);
+    return hipGetLastError();
+  }
   const int small = quad_sadj_small_doubles(Q.k, Q.l);
   const int full = small + 3 * quad_sadj_r3(Q.k, Q.l) + Q.l * Q.l * Q.l;
   if (full <= kSAdjLdsMax)
