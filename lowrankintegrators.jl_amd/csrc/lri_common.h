@@ -39,6 +39,27 @@ __device__ __forceinline__ void split_bf16(float x, uint32_t& hi, uint32_t& lo) 
   lo = f32_to_bf16_rne(r);
 }
 
+// ---------------------------------------------------------------- reciprocals
+// 1/sqrt(d) for normal d > 0: the hardware estimate refined by two Newton
+// steps y <- y + y (1 - d y^2) / 2.
+__device__ __forceinline__ double rsqrt_nr(double d) {
+  double y = __builtin_amdgcn_rsq(d);
+  double r = __builtin_fma(-d * y, y, 1.0);
+  y = __builtin_fma(0.5 * y, r, y);
+  r = __builtin_fma(-d * y, y, 1.0);
+  return __builtin_fma(0.5 * y, r, y);
+}
+
+// 1/d for normal d: the hardware estimate refined by two Newton steps
+// y <- y + y (1 - d y).
+__device__ __forceinline__ double rcp_nr(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  double r = __builtin_fma(-d, y, 1.0);
+  y = __builtin_fma(y, r, y);
+  r = __builtin_fma(-d, y, 1.0);
+  return __builtin_fma(y, r, y);
+}
+
 // ---------------------------------------------------------------- small products on the matrix cores
 // C(m, n) = sum_kk A(b, m, kk) B(b, kk, n) for b < nbatch, in 16 x 16 blocks
 // distributed over the workgroup's waves (v_mfma_f64_16x16x4_f64: lane l holds

@@ -497,7 +497,172 @@ hipError_t launch_spectral_flow(double* Z, int64_t n, int k, const double* lam, 
 }
 
 // ----------------------------------------------------------------------------
-// Symmetric k x k eigen-decomposition (k <= 128) as the one-sided Jacobi SVD of
+// Symmetric k x k eigen-decomposition for k <= 64: cyclic two-sided Jacobi in one
+// workgroup.  The pairs of a round are disjoint and pair I's rotation comes from
+// the 2 x 2 block of the matrix at (I, I), so a round is one read of the matrix and
+// of the accumulated rotations, one serial chain of about twenty FP64 operations
+// and one write.  What bounds it is the issue of its instructions (four cycles each
+// for a wave), so the pairs always sit in the same places, rows and columns 2 I and
+// 2 I + 1: a round writes its results where the next round of the tournament wants
+// them (positions move by seat_after), into a second buffer, so that every address is
+// computed once, blocks are read 16 bytes at a time and one barrier a round is enough.
+// Thread (I, J) of kP x kP updates block (I, J) and the rows I, I + kP of V in
+// pair J's columns.  It computes the rotations of both pairs itself (for kP = 32, where
+// the 16 waves fill the SIMDs, that of I only and takes J's from lane J).
+// The one-sided form on M + sigma I before (sums over whole columns for every
+// rotation, one wave, preceded by a QR and a shift, followed by an unshift) took
+// 308 us for two matrices of k = 32 (and 9 us for the two small launches), this one
+// 126 to 150 us (eight or nine sweeps of 31 rounds); a batched launch of pairs with k <= 56
+// went from 956 to 474 us.
+// M is scaled by a power of two to norm 1 (largest row sum); pairs rotate while
+// |m_pq| > eps / 64 of that norm.
+// ----------------------------------------------------------------------------
+
+// The rotation (c, s) that annihilates m_pq, if m_pq^2 > thr:
+// tan = sign(h) 2 m_pq / (|h| + sqrt(h^2 + 4 m_pq^2)), h = m_qq - m_pp, from the hardware's
+// reciprocal and square-root estimates (the next sweep sees what they leave of
+// m_pq); c and s = c tan are orthonormal to rounding.
+__device__ __forceinline__ bool sym_rotation(double app, double apq, double aqq, double thr, double& c, double& s) {
+  const double h = aqq - app, g2 = 2.0 * apq;
+  const double q = __builtin_fma(h, h, g2 * g2);
+  double tt = g2 * __builtin_amdgcn_rcp(fabs(h) + q * __builtin_amdgcn_rsq(q));
+  if (h < 0.0) tt = -tt;
+  const bool rot = apq * apq > thr;
+  tt = rot ? tt : 0.0;
+  c = rsqrt_nr(__builtin_fma(tt, tt, 1.0));
+  s = c * tt;
+  return rot;
+}
+
+// The next seat of the player in seat x of a round-robin tournament of np tables
+// (seats 2 i and 2 i + 1): seat 0 stays, the others move round; 2 np - 1 rounds bring
+// everybody back.
+__device__ __forceinline__ int seat_after(int x, int np) {
+  const int i = x >> 1;
+  if (np == 1 || x == 0) return x;
+  if (x & 1) return i == 0 ? 2 : x - 2;
+  return i == np - 1 ? x + 1 : x + 2;
+}
+
+template <int kP>  // k <= 2 kP; kP^2 threads
+__device__ __forceinline__ void sym_eig_body(const SymEigArgs& Q) {
+  constexpr int kN = 2 * kP, kLd = kN + 2, kSize = kN * kLd;
+  // the matrix, column-major, and V, row-major, twice each
+  __shared__ __attribute__((aligned(16))) double A[2 * kSize], V[2 * kSize];
+  __shared__ double sums[kN];
+  __shared__ int pos[kN];
+  const int t = threadIdx.x, k = Q.k;
+  for (int e = t; e < kN * kN; e += kP * kP) {
+    const int i = e % kN, j = e / kN;
+    // symmetrised (the Galerkin products are symmetric up to rounding)
+    A[i + j * kLd] = i < k && j < k ? 0.5 * (Q.M[i + j * Q.ldm] + Q.M[j + i * Q.ldm]) : 0.0;
+    V[i + j * kLd] = i == j ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  if (t < kN) {
+    double s = 0.0;
+    for (int j = 0; j < k; ++j) s += fabs(A[t + j * kLd]);
+    sums[t] = s;
+  }
+  __syncthreads();
+  double norm = 0.0;
+  for (int j = 0; j < kN; ++j) norm = fmax(norm, sums[j]);
+  int ex = 0;
+  if (norm > 0.0 && isfinite(norm)) frexp(norm, &ex);
+  for (int e = t; e < kN * kN; e += kP * kP) {
+    const int o = e % kN + (e / kN) * kLd;
+    A[o] = ldexp(A[o], -ex);
+  }
+  const int np = (k + 1) / 2;
+  const int I = t % kP, J = t / kP;
+  const bool actI = I < np, act = actI && J < np;
+  constexpr double kThr = 2.220446049250313e-16 * 2.220446049250313e-16 / 4096.0;
+  // where this thread reads, and where its results go in the other buffer
+  const int rIJ = 2 * I + 2 * J * kLd, rII = 2 * I * (kLd + 1), rJJ = 2 * J * (kLd + 1);
+  const int rV = I * kLd + 2 * J, rV2 = rV + kP * kLd;
+  const int pI = seat_after(2 * I, np), qI = seat_after(2 * I + 1, np);
+  const int pJ = seat_after(2 * J, np), qJ = seat_after(2 * J + 1, np);
+  const int wa = pI + pJ * kLd, wb = pI + qJ * kLd, wc = qI + pJ * kLd, wd = qI + qJ * kLd;
+  const int wv = I * kLd + pJ, ww = I * kLd + qJ;
+  typedef __attribute__((ext_vector_type(2))) double f64x2;
+  auto two = [](const double* p) { return *reinterpret_cast<const f64x2*>(p); };
+  __syncthreads();
+  int cur = 0;
+  for (int sweep = 0; sweep < 40; ++sweep) {
+    int rot = 0;
+    for (int r = 0; r < 2 * np - 1; ++r) {
+      const double* Ar = A + cur;
+      const double* Vr = V + cur;
+      cur = kSize - cur;
+      double* Aw = A + cur;
+      double* Vw = V + cur;
+      const f64x2 dI = two(Ar + rII), eI = two(Ar + rII + kLd);  // (pp, qp), (pq, qq)
+      const f64x2 dJ = kP <= 16 ? two(Ar + rJJ) : dI, eJ = kP <= 16 ? two(Ar + rJJ + kLd) : eI;
+      const f64x2 ac = two(Ar + rIJ), bd = two(Ar + rIJ + kLd);
+      const f64x2 v0 = two(Vr + rV), v1 = two(Vr + rV2);
+      double cI, sI, cJ, sJ;
+      const bool ro = sym_rotation(dI[0], eI[0], eI[1], kThr, cI, sI);
+      rot |= (int)(actI & ro);
+      if (kP <= 16) {
+        sym_rotation(dJ[0], eJ[0], eJ[1], kThr, cJ, sJ);
+      } else {  // lane J holds pair J's
+        cJ = __shfl(cI, J);
+        sJ = __shfl(sI, J);
+      }
+      if (act) {
+        const double a1 = cI * ac[0] - sI * ac[1], c1 = sI * ac[0] + cI * ac[1];
+        const double b1 = cI * bd[0] - sI * bd[1], d1 = sI * bd[0] + cI * bd[1];
+        Aw[wa] = cJ * a1 - sJ * b1;
+        Aw[wb] = sJ * a1 + cJ * b1;
+        Aw[wc] = cJ * c1 - sJ * d1;
+        Aw[wd] = sJ * c1 + cJ * d1;
+      }
+      if (J < np) {
+        Vw[wv] = cJ * v0[0] - sJ * v0[1];
+        Vw[ww] = sJ * v0[0] + cJ * v0[1];
+        Vw[wv + kP * kLd] = cJ * v1[0] - sJ * v1[1];
+        Vw[ww + kP * kLd] = sJ * v1[0] + cJ * v1[1];
+      }
+      __syncthreads();
+    }
+    if (!__syncthreads_or(rot)) break;
+  }
+  const double* Af = A + cur;
+  const double* Vf = V + cur;
+  if (t < k) {  // descending eigenvalues
+    const double ev = Af[t + t * kLd];
+    int at = 0;
+    for (int l = 0; l < k; ++l) {
+      const double o = Af[l + l * kLd];
+      at += o > ev || (o == ev && l < t);
+    }
+    pos[t] = at;
+    Q.ev[at] = ldexp(ev, ex);
+  }
+  __syncthreads();
+  for (int e = t; e < k * k; e += kP * kP) {
+    const int i = e % k, j = e / k;
+    Q.W[i + pos[j] * k] = Vf[i * kLd + j];
+  }
+}
+
+struct SymEigPair {
+  SymEigArgs P0, P1;
+};
+template <int kP>
+__global__ __launch_bounds__(kP* kP) void k_sym_eig(SymEigPair S) {
+  sym_eig_body<kP>(blockIdx.x == 0 ? S.P0 : S.P1);
+}
+template <int kP>
+__global__ __launch_bounds__(kP* kP) void k_sym_eig_batch(const unsigned char* __restrict__ tab,
+                                                          const int* __restrict__ start, int count) {
+  const int i = batch_member(start, count, blockIdx.x);
+  const SymEigPair& S = *reinterpret_cast<const SymEigPair*>(tab + (size_t)start[count + 1 + i] * kRecArgBytes);
+  sym_eig_body<kP>(blockIdx.x - start[i] == 0 ? S.P0 : S.P1);
+}
+
+// ----------------------------------------------------------------------------
+// The same for 64 < k <= 128 as the one-sided Jacobi SVD of
 // M + sigma I with sigma = max_i sum_j |M_ij| >= spectral radius, so the
 // shifted matrix is positive semidefinite: its singular vectors are
 // eigenvectors of M and its singular values minus sigma the eigenvalues.
@@ -574,11 +739,26 @@ __global__ void k_unshift_batch(const unsigned char* __restrict__ tab, const int
 
 hipError_t launch_sym_eig(const SymEigArgs* P, int count, hipStream_t st) {
   if (count < 1 || count > 2) return hipErrorInvalidValue;
+  int kmax = 0;
+  for (int b = 0; b < count; ++b) {
+    if (P[b].k < 1 || P[b].k > kMaxAug) return hipErrorInvalidValue;
+    kmax = std::max(kmax, P[b].k);
+  }
+  if (kmax <= 64) {
+    const SymEigPair S{P[0], P[count - 1]};
+    const int half = kmax <= 16 ? 8 : kmax <= 32 ? 16 : 32;
+    if (!record_launch(KID_SYM_EIG, half, (unsigned)count, (unsigned)(half * half), 0, S)) {
+      const dim3 g(count), t(half * half);
+      if (half == 8) hipLaunchKernelGGL(k_sym_eig<8>, g, t, 0, st, S);
+      else if (half == 16) hipLaunchKernelGGL(k_sym_eig<16>, g, t, 0, st, S);
+      else hipLaunchKernelGGL(k_sym_eig<32>, g, t, 0, st, S);
+    }
+    return hipGetLastError();
+  }
   ShiftArgs sa[2];
   SvdArgs sv[2];
   for (int b = 0; b < count; ++b) {
     const SymEigArgs& p = P[b];
-    if (p.k < 1 || p.k > kMaxAug) return hipErrorInvalidValue;
     sa[b] = ShiftArgs{p.M, p.ldm, p.k, p.work, p.work + (size_t)p.k * p.k, p.ev};
     sv[b].S = p.work;
     sv[b].lds = p.k;
@@ -624,6 +804,11 @@ hipError_t launch_de_batched(int kid, int variant, const void* tab, const int* s
       else hipLaunchKernelGGL(k_s_substep_batch<false>, g, b, lds, st, t, start, count);
       break;
     case KID_FLOW: hipLaunchKernelGGL(k_spectral_flow_batch, g, b, lds, st, t, start, count); break;
+    case KID_SYM_EIG:
+      if (variant == 8) hipLaunchKernelGGL(k_sym_eig_batch<8>, g, b, lds, st, t, start, count);
+      else if (variant == 16) hipLaunchKernelGGL(k_sym_eig_batch<16>, g, b, lds, st, t, start, count);
+      else hipLaunchKernelGGL(k_sym_eig_batch<32>, g, b, lds, st, t, start, count);
+      break;
     case KID_SHIFT: hipLaunchKernelGGL(k_shift_sym_batch, g, b, lds, st, t, start, count); break;
     case KID_UNSHIFT: hipLaunchKernelGGL(k_unshift_batch, g, b, lds, st, t, start, count); break;
     default: return hipErrorInvalidValue;

@@ -28,6 +28,7 @@ enum KernelId : int {
   KID_EPILOGUE,     // k_epilogue<CK>; variant = CK
   KID_JACOBI_WAVE,  // k_jacobi_wave (two decompositions per record)
   KID_JACOBI_WG,    // k_jacobi_svd
+  KID_SYM_EIG,      // k_sym_eig<kP> (one or two decompositions per record); variant = kP
   KID_SHIFT,        // k_shift_sym
   KID_UNSHIFT,      // k_unshift
   KID_DE_PREP,      // k_de_prep<kLds>; variant = kLds

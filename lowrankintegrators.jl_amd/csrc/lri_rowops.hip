@@ -41,26 +41,6 @@ __device__ __forceinline__ double readlane_f64(double x, int lane) {
   return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
 }
 
-// 1/sqrt(d) for normal d > 0: the hardware estimate refined by two Newton
-// steps y <- y + y (1 - d y^2) / 2.
-__device__ __forceinline__ double rsqrt_nr(double d) {
-  double y = __builtin_amdgcn_rsq(d);
-  double r = __builtin_fma(-d * y, y, 1.0);
-  y = __builtin_fma(0.5 * y, r, y);
-  r = __builtin_fma(-d * y, y, 1.0);
-  return __builtin_fma(0.5 * y, r, y);
-}
-
-// 1/d for normal d: the hardware estimate refined by two Newton steps
-// y <- y + y (1 - d y).
-__device__ __forceinline__ double rcp_nr(double d) {
-  double y = __builtin_amdgcn_rcp(d);
-  double r = __builtin_fma(-d, y, 1.0);
-  y = __builtin_fma(y, r, y);
-  r = __builtin_fma(-d, y, 1.0);
-  return __builtin_fma(y, r, y);
-}
-
 // Exponent e (even) with max_diag * 2^-e in [0.5, 2): the Gram matrix is
 // scaled by 2^-e (exactly), so R scales by 2^(-e/2) and every pivot stays a
 // normal number; zero, NaN and Inf give 0.
