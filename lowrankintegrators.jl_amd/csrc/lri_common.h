@@ -13,7 +13,7 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 namespace lri {
 
 // Device-side status bits latched into ctx->flags (read at synchronising calls).
-enum : int { FLAG_BREAKDOWN = 1, FLAG_NONFINITE = 2 };
+enum : int { FLAG_BREAKDOWN = 1, FLAG_NONFINITE = 2, FLAG_TIMEOUT = 4 };
 
 constexpr int kMaxRank = 64;       // state rank capacity
 constexpr int kMaxAug = 2 * kMaxRank;  // rank-adaptive augmented width

@@ -676,6 +676,72 @@ struct lri_ctx {
     rows(C);
   }
 
+  // The matrix of the next qr(): its formation as row-kernel arguments (out = X), or
+  // X itself.
+  RowArgs<double> held_d;
+  RowArgs<float> held_f;
+  bool held_f32 = false;
+  void hold(const RowArgs<double>& A) {
+    held_d = A;
+    held_f32 = false;
+  }
+  void hold(const RowArgs<float>& A) {
+    held_f = A;
+    held_f32 = true;
+  }
+  void hold_matrix(const double* X, int64_t rows_, int k) {
+    RowArgs<double> A;
+    A.rows = rows_;
+    A.r_out = k;
+    A.base = X;
+    A.ld_base = rows_;
+    hold(A);
+  }
+  // The CholeskyQR2 (passes = 3: shifted CholeskyQR3) of the held matrix into `out`, Rtot in
+  // small: one launch where it fits (k_qr), else rows() and cholqr_tail, whose arguments
+  // the others are (first: the EPI_CHOL1 arguments).  Recorded steps (a batch's merged
+  // launches) take the separate kernels: k_qr's workgroups wait for each other, and a merged
+  // launch over hundreds of members does not keep them resident together.
+  void qr(const EpiArgs& first, double* X, double* tmp, int64_t rows_, int rr, double* out, bool pk_forN,
+          const double* W, const EpiArgs& fin, int sfinal, int passes) {
+    if (held_f32) qr_of(held_f, first, X, tmp, rows_, rr, out, pk_forN, W, fin, sfinal, passes);
+    else qr_of(held_d, first, X, tmp, rows_, rr, out, pk_forN, W, fin, sfinal, passes);
+  }
+  template <typename PT>
+  void qr_of(RowArgs<PT> A, const EpiArgs& first, double* X, double* tmp, int64_t rows_, int rr, double* out,
+             bool pk_forN, const double* W, const EpiArgs& fin, int sfinal, int passes) {
+    if (current_recorder() || !qr_fits(rows_, rr, passes)) {
+      const bool fold = fold_chol(rr, passes);
+      A.reduce = 1;
+      A.epi = first;
+      A.defer_epi = fold;
+      rows(A);
+      cholqr_tail(X, tmp, rows_, rr, out, pk_forN, W, W ? rr : 0, fin, sfinal, passes, fold ? &first : nullptr);
+      return;
+    }
+    QrArgs<PT> Q;
+    set_pack_outputs(A, pk_forN, pass_mode(), rb_for(pass_mode(), rr));
+    Q.form = A;
+    Q.q = out;
+    Q.passes = passes;
+    Q.shift_rows = first.shift_rows;
+    Q.first_error = first.breakdown_is_error;
+    Q.later_error = fin.breakdown_is_error;
+    Q.S = sfinal ? S : nullptr;
+    Q.ld_s = (int)rcap;
+    Q.transpose_s = sfinal == 2;
+    Q.W = W;
+    Q.ldw = rows_;
+    if (passes == 2 && W && fin.kind == EPI_STILDE) Q.stilde = fin.transpose ? 2 : 1;  // with the second factor
+    else Q.fin = fin;
+    Q.small = Q.fin.small = small;
+    Q.fin.flags = flags;
+    Q.gpart = gpart;
+    Q.sync = flags + 8;
+    Q.flags = flags;
+    timed(LRI_KERNEL_SMALL, [&] { return launch_qr(Q, stream); });
+  }
+
   // After a KSL CholeskyQR2 of X (rows_ x rr) into Q: when a pivot was dropped
   // (a rank-deficient K or L), the QR is recomputed from X by reorthogonalised
   // Gram-Schmidt with an orthonormal completion, as Householder QR (qr! in
@@ -729,7 +795,6 @@ struct lri_ctx {
   // primal_LT_step! (projector_splitting.jl:129-152)
   void ksl_primal(int64_t kp, int64_t kn) {
     const int rr = (int)r;
-    const bool fold = fold_chol(rr);
     EpiArgs c1;
     c1.kind = EPI_CHOL1;
     c1.breakdown_is_error = 0;  // dropped columns are completed
@@ -749,15 +814,12 @@ struct lri_ctx {
       A.ldy = (int)rcap;
       A.out = K;
       A.ldo = n;
-      A.reduce = 1;
-      A.epi = c1;
-      A.defer_epi = fold;
-      rows(A);
+      hold(A);
     });
     EpiArgs e;
     e.kind = EPI_STILDE;  // S~ = R - U1' P
     e.breakdown_is_error = 0;
-    cholqr_tail(K, K2, n, rr, U, false, P, rr, e, 0, 2, fold ? &c1 : nullptr);
+    qr(c1, K, K2, n, rr, U, false, P, e, 0, 2);
     complete_dropped(K, U, n, rr, false, small->St, rr, 0, P, n, nullptr, 0, 0);  // S~ = R - U1' P
     const int sT = passT(kp, kn, rr, partT);
     with_parts(partT, [&](auto A) {  // L = V S~' + dA' U1 ; Gram -> R1
@@ -773,21 +835,17 @@ struct lri_ctx {
       A.transY = 1;
       A.out = L;
       A.ldo = m;
-      A.reduce = 1;
-      A.epi = c1;
-      A.defer_epi = fold;
-      rows(A);
+      hold(A);
     });
     EpiArgs none;
     none.breakdown_is_error = 0;
-    cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 2, 2, fold ? &c1 : nullptr);  // V1, S = R'
+    qr(c1, L, L2, m, rr, V, true, nullptr, none, 2, 2);  // V1, S = R'
     complete_dropped(L, V, m, rr, true, nullptr, 0, 0, nullptr, 0, S, (int)rcap, 1);  // S = R'
   }
 
   // dual_LT_step! (projector_splitting.jl:166-189)
   void ksl_dual(int64_t kp, int64_t kn) {
     const int rr = (int)r;
-    const bool fold = fold_chol(rr);
     EpiArgs c1;
     c1.kind = EPI_CHOL1;
     c1.breakdown_is_error = 0;  // dropped columns are completed
@@ -808,16 +866,13 @@ struct lri_ctx {
       A.transY = 1;
       A.out = L;
       A.ldo = m;
-      A.reduce = 1;
-      A.epi = c1;
-      A.defer_epi = fold;
-      rows(A);
+      hold(A);
     });
     EpiArgs e;
     e.kind = EPI_STILDE;  // S~ = (R - V1' Q)' = R' - U' dA V1
     e.transpose = 1;
     e.breakdown_is_error = 0;
-    cholqr_tail(L, L2, m, rr, V, true, Q, rr, e, 0, 2, fold ? &c1 : nullptr);
+    qr(c1, L, L2, m, rr, V, true, Q, e, 0, 2);
     complete_dropped(L, V, m, rr, true, small->St, rr, 1, Q, m, nullptr, 0, 0);  // S~ = (R - V1' Q)'
     const int sN = passN(kp, kn, rr, partN);
     with_parts(partN, [&](auto A) {  // K = U S~ + dA V1
@@ -832,21 +887,17 @@ struct lri_ctx {
       A.ldy = rr;
       A.out = K;
       A.ldo = n;
-      A.reduce = 1;
-      A.epi = c1;
-      A.defer_epi = fold;
-      rows(A);
+      hold(A);
     });
     EpiArgs none;
     none.breakdown_is_error = 0;
-    cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 1, 2, fold ? &c1 : nullptr);  // U1, S = R
+    qr(c1, K, K2, n, rr, U, false, nullptr, none, 1, 2);  // U1, S = R
     complete_dropped(K, U, n, rr, false, nullptr, 0, 0, nullptr, 0, S, (int)rcap, 0);  // S = R
   }
 
   // unconventional_step! (unconventional.jl:133-157)
   void bug(int64_t kp, int64_t kn) {
     const int rr = (int)r;
-    const bool fold = fold_chol(rr);
     EpiArgs c1;
     c1.kind = EPI_CHOL1;
     ensure_packed(true);
@@ -865,14 +916,11 @@ struct lri_ctx {
       A.ldy = (int)rcap;
       A.out = K;
       A.ldo = n;
-      A.reduce = 1;
-      A.epi = c1;
-      A.defer_epi = fold;
-      rows(A);
+      hold(A);
     });
     EpiArgs eM;
     eM.kind = EPI_BUG_M;  // M = U1' U0
-    cholqr_tail(K, K2, n, rr, U2, false, U, rr, eM, 0, 2, fold ? &c1 : nullptr);
+    qr(c1, K, K2, n, rr, U2, false, U, eM, 0, 2);
     with_parts(partT, [&](auto A) {
       A.rows = m;
       A.nsplit = sT;
@@ -886,16 +934,13 @@ struct lri_ctx {
       A.transY = 1;
       A.out = L;
       A.ldo = m;
-      A.reduce = 1;
-      A.epi = c1;
-      A.defer_epi = fold;
-      rows(A);
+      hold(A);
     });
     EpiArgs eN;
     eN.kind = EPI_BUG_N;  // N = V1' V0, Sinit = M S0 N'
     eN.S = S;
     eN.ld_s = (int)rcap;
-    cholqr_tail(L, L2, m, rr, V2, true, V, rr, eN, 0, 2, fold ? &c1 : nullptr);
+    qr(c1, L, L2, m, rr, V2, true, V, eN, 0, 2);
     const int sN2 = passN(kp, kn, rr, partN);  // dA V1
     with_parts(partN, [&](auto A) {  // S1 = Sinit + U1' dA V1
       A.rows = n;
@@ -935,11 +980,9 @@ struct lri_ctx {
       A.r_out = rr;
       A.out = K;
       A.ldo = n;
-      A.reduce = 1;
-      A.epi = shifted_chol(n);
-      rows(A);
+      hold(A);
     });
-    cholqr_tail(K, K2, n, rr, U2, false, nullptr, 0, none, 0, 3);  // U1 (packed for pass T)
+    qr(shifted_chol(n), K, K2, n, rr, U2, false, nullptr, none, 0, 3);  // U1 (packed for pass T)
     with_parts(partT, [&](auto A) {
       A.rows = m;
       A.nsplit = sT;
@@ -947,11 +990,9 @@ struct lri_ctx {
       A.r_out = rr;
       A.out = L;
       A.ldo = m;
-      A.reduce = 1;
-      A.epi = shifted_chol(m);
-      rows(A);
+      hold(A);
     });
-    cholqr_tail(L, L2, m, rr, V2, true, nullptr, 0, none, 0, 3);  // V1 (packed for pass N)
+    qr(shifted_chol(m), L, L2, m, rr, V2, true, nullptr, none, 0, 3);  // V1 (packed for pass N)
     const int sN2 = passN(-1, kn, rr, partN);  // X V1
     with_parts(partN, [&](auto A) {  // C = (X V1)' U1 = S1'
       A.rows = n;
@@ -1014,7 +1055,7 @@ struct lri_ctx {
     } else {
       de_galerkin(U, true, rr, de->Ga, de->gaT);       // U'AU, G'U
       de_eig(de->Ga, rr, de->Wa, de->alpha);
-      de_substep(V, false, rr, de->Snew, rr, 1, de->Wa, de->alpha, de->gaT, h, nsub, V, L2, de_epi());
+      de_substep(V, false, rr, de->Snew, rr, 1, de->Wa, de->alpha, de->gaT, h, nsub, V, L2, false);
     }
     pack_enabled = true;
     pkN_mode = pkT_mode = -1;
@@ -1037,11 +1078,9 @@ struct lri_ctx {
       A.r_out = rr;
       A.out = K;
       A.ldo = n;
-      A.reduce = 1;
-      A.epi = shifted_chol(n);
-      rows(A);
+      hold(A);
     });
-    cholqr_tail(K, K2, n, rr, U2, false, nullptr, 0, none, 0, 3);  // Qc, R = Rtot
+    qr(shifted_chol(n), K, K2, n, rr, U2, false, nullptr, none, 0, 3);  // Qc, R = Rtot
     SvdArgs sv;
     sv.S = small->Rtot;
     sv.lds = rr;
@@ -1086,6 +1125,8 @@ struct lri_ctx {
     const int mode = pass_mode();
     const int rb = rb_for(mode, rr);
     const size_t rsz = sizeof(double) * rr * rr;
+    EpiArgs c1;
+    c1.kind = EPI_CHOL1;
     // forward: K1 = U0 S0 + dA V0 -> U1, RK ; L1 = V0 S0' + dA' U0 -> V1, RL ; M, N
     ensure_packed(true);
     ensure_packed(false);
@@ -1103,13 +1144,11 @@ struct lri_ctx {
       A.ldy = (int)rcap;
       A.out = K;
       A.ldo = n;
-      A.reduce = 1;
-      A.epi.kind = EPI_CHOL1;
-      rows(A);
+      hold(A);
     });
     EpiArgs eM;
     eM.kind = EPI_BUG_M;  // M = U1' U0
-    cholqr_tail(K, K2, n, rr, U2, false, U, rr, eM, 0);
+    qr(c1, K, K2, n, rr, U2, false, U, eM, 0, 2);
     HIPCHECK(hipMemcpyAsync(adj->RK, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
     with_parts(partT, [&](auto A) {
       A.rows = m;
@@ -1124,14 +1163,12 @@ struct lri_ctx {
       A.transY = 1;
       A.out = L;
       A.ldo = m;
-      A.reduce = 1;
-      A.epi.kind = EPI_CHOL1;
-      rows(A);
+      hold(A);
     });
     EpiArgs eNs;
     eNs.kind = EPI_COPY;  // N = V1' V0
     eNs.dst = small->N;
-    cholqr_tail(L, L2, m, rr, V2, true, V, rr, eNs, 0);
+    qr(c1, L, L2, m, rr, V2, true, V, eNs, 0, 2);
     HIPCHECK(hipMemcpyAsync(adj->RL, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
     timed(LRI_KERNEL_SMALL, [&] { return launch_bug_adj_pre(adj, small->M, small->N, S, (int)rcap, rr, stream); });
     double* Ub = P;           // in: Ub1, out: Ub0
@@ -1286,6 +1323,8 @@ struct lri_ctx {
     const int mode = pass_mode();
     const int rb = rb_for(mode, rr);
     const size_t rsz = sizeof(double) * rr * rr;
+    EpiArgs c1;
+    c1.kind = EPI_CHOL1;
     ensure_packed(true);
     const int sN = passN(kp, kn, rr, partN);
     with_parts(partN, [&](auto A) {  // K = U S + dA V ; P = dA V ; Gram -> R1
@@ -1302,13 +1341,11 @@ struct lri_ctx {
       A.ldy = (int)rcap;
       A.out = K;
       A.ldo = n;
-      A.reduce = 1;
-      A.epi.kind = EPI_CHOL1;
-      rows(A);
+      hold(A);
     });
     EpiArgs e;
     e.kind = EPI_STILDE;  // S~ = R - U1' P
-    cholqr_tail(K, K2, n, rr, U2, false, P, rr, e, 0);  // U1 (packed for pass T)
+    qr(c1, K, K2, n, rr, U2, false, P, e, 0, 2);  // U1 (packed for pass T)
     HIPCHECK(hipMemcpyAsync(adj->RK, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
     HIPCHECK(hipMemcpyAsync(adj->St, small->St, rsz, hipMemcpyDeviceToDevice, stream));
     const int sT = passT(kp, kn, rr, partT);
@@ -1325,12 +1362,10 @@ struct lri_ctx {
       A.transY = 1;
       A.out = L;
       A.ldo = m;
-      A.reduce = 1;
-      A.epi.kind = EPI_CHOL1;
-      rows(A);
+      hold(A);
     });
     EpiArgs none;
-    cholqr_tail(L, L2, m, rr, V2, true, nullptr, 0, none, 0);  // V1
+    qr(c1, L, L2, m, rr, V2, true, nullptr, none, 0, 2);  // V1
     HIPCHECK(hipMemcpyAsync(adj->RL, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
     timed(LRI_KERNEL_SMALL, [&] { return launch_ksl_adj_small(adj, rr, 0, stream); });
     double* Ub = P + n * rr;   // P[:, :r] holds dA V0; the cotangents sit in the next r columns
@@ -2324,7 +2359,7 @@ struct lri_ctx {
     }
   }
 
-  void de_finish(bool nside, int k, const double* Wo, double* out, const double* scratch, EpiArgs epi) {
+  RowArgs<double> de_finish_args(bool nside, int k, const double* Wo, double* out, const double* scratch) {
     const int64_t rows_ = nside ? n : m;
     RowArgs<double> B;  // Z = Zbar Wo'
     B.rows = rows_;
@@ -2337,17 +2372,19 @@ struct lri_ctx {
     B.transY = 1;
     B.out = out;
     B.ldo = rows_;
-    if (epi.kind != EPI_NONE) {
-      B.reduce = 1;
-      B.epi = epi;
-    }
-    rows(B);
+    return B;
   }
+  void de_finish_hold(bool nside, int k, const double* Wo, double* out, const double* scratch) {
+    hold(de_finish_args(nside, k, Wo, out, scratch));
+  }
+  // hold_result: Z is left to the next qr() (hold), else formed
   void de_substep(const double* X0, bool nside, int k, const double* C0, int ldc, int transC, const double* Wo,
                   const double* ev, const double* FXo, double h, int64_t nsub, double* out, double* scratch,
-                  EpiArgs epi) {
+                  bool hold_result) {
     de_run(de_prepare(X0, nside, k, C0, ldc, transC, Wo, ev, FXo, 0, h, nsub, scratch));
-    de_finish(nside, k, Wo, out, scratch, epi);
+    const RowArgs<double> B = de_finish_args(nside, k, Wo, out, scratch);
+    if (hold_result) hold(B);
+    else rows(B);
   }
   void de_sstep(int k, int l, const double* S0, int lds0, int transS0, double* S1, int lds1, double sgn, double h,
                 int64_t nsub) {
@@ -2516,17 +2553,6 @@ struct lri_ctx {
     B.store = stL;
     quad_steps(A, K, work, B, L, work + std::max(n, m) * k, nsub);
   }
-  // Gram of X (rows x k) and the shifted first CholeskyQR factor
-  void quad_gram(const double* X, int64_t rows_, int k, EpiArgs epi) {
-    RowArgs<double> A;
-    A.rows = rows_;
-    A.r_out = k;
-    A.base = X;
-    A.ld_base = rows_;
-    A.reduce = 1;
-    A.epi = epi;
-    rows(A);
-  }
   void quad_sstep(int k, const double* S0, int lds0, int transS0, double* S1, int lds1, double sgn, double h,
                   int64_t nsub) {
     QuadSArgs Q;
@@ -2556,14 +2582,14 @@ struct lri_ctx {
     quad_galerkin(V, false, rr);  // V0'BV0, H'V0, T(V0)
     quad_init(U, n, rr, S, (int)rcap, 0, K);
     quad_rows(true, rr, K, K2, h, nsub);
-    quad_gram(K, n, rr, shifted_chol(n));
-    cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 0, 3);  // U1, R
+    hold_matrix(K, n, rr);
+    qr(shifted_chol(n), K, K2, n, rr, U, false, nullptr, none, 0, 3);  // U1, R
     quad_galerkin(U, true, rr);                                    // U1'AU1, G'U1, W(U1)
     quad_sstep(rr, small->Rtot, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
     quad_init(V, m, rr, de->Snew, rr, 1, L);
     quad_rows(false, rr, L, L2, h, nsub);
-    quad_gram(L, m, rr, shifted_chol(m));
-    cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 2, 3);  // V1, S = R'
+    hold_matrix(L, m, rr);
+    qr(shifted_chol(m), L, L2, m, rr, V, true, nullptr, none, 2, 3);  // V1, S = R'
   }
 
   void quad_ksl_dual(double dt, int64_t nsub) {
@@ -2573,14 +2599,14 @@ struct lri_ctx {
     quad_galerkin(U, true, rr);  // U0'AU0, G'U0, W(U0)
     quad_init(V, m, rr, S, (int)rcap, 1, L);
     quad_rows(false, rr, L, L2, h, nsub);
-    quad_gram(L, m, rr, shifted_chol(m));
-    cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 0, 3);  // V1, R
+    hold_matrix(L, m, rr);
+    qr(shifted_chol(m), L, L2, m, rr, V, true, nullptr, none, 0, 3);  // V1, R
     quad_galerkin(V, false, rr);                                  // V1'BV1, H'V1, T(V1)
     quad_sstep(rr, small->Rtot, rr, 1, de->Snew, rr, -1.0, h, nsub);  // S~ from R'
     quad_init(U, n, rr, de->Snew, rr, 0, K);
     quad_rows(true, rr, K, K2, h, nsub);
-    quad_gram(K, n, rr, shifted_chol(n));
-    cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 1, 3);  // U1, S = R
+    hold_matrix(K, n, rr);
+    qr(shifted_chol(n), K, K2, n, rr, U, false, nullptr, none, 1, 3);  // U1, S = R
   }
 
   void quad_bug(double dt, int64_t nsub) {
@@ -2592,13 +2618,13 @@ struct lri_ctx {
     }
     de_gal_fresh = false;
     quad_rows_pair(rr, h, nsub);
-    quad_gram(K, n, rr, shifted_chol(n));
-    cholqr_tail(K, K2, n, rr, U2, false, U, rr, de_epi(EPI_BUG_M), 0, 3);  // U1, M = U1'U0
-    quad_gram(L, m, rr, shifted_chol(m));
+    hold_matrix(K, n, rr);
+    qr(shifted_chol(n), K, K2, n, rr, U2, false, U, de_epi(EPI_BUG_M), 0, 3);  // U1, M = U1'U0
+    hold_matrix(L, m, rr);
     EpiArgs eN = de_epi(EPI_BUG_N);  // N = V1'V0, Sinit = M S0 N'
     eN.S = S;
     eN.ld_s = (int)rcap;
-    cholqr_tail(L, L2, m, rr, V2, true, V, rr, eN, 0, 3);
+    qr(shifted_chol(m), L, L2, m, rr, V2, true, V, eN, 0, 3);
     quad_galerkin(U2, true, rr);
     quad_galerkin(V2, false, rr);
     quad_sstep(rr, small->Sinit, rr, 0, S, (int)rcap, 1.0, h, nsub);
@@ -2761,14 +2787,14 @@ struct lri_ctx {
     HIPCHECK(hipMemcpyAsync(qa->W0, quad_W, tsz, hipMemcpyDeviceToDevice, stream));
     HIPCHECK(hipMemcpyAsync(qa->T0, quad_T, tsz, hipMemcpyDeviceToDevice, stream));
     quad_rows_pair_kept(rr, work, stK, stL, h, nsub);
-    quad_gram(K, n, rr, shifted_chol(n));
-    cholqr_tail(K, K2, n, rr, U2, false, U, rr, de_epi(EPI_BUG_M), 0, 3);  // U1, M = U1'U0
+    hold_matrix(K, n, rr);
+    qr(shifted_chol(n), K, K2, n, rr, U2, false, U, de_epi(EPI_BUG_M), 0, 3);  // U1, M = U1'U0
     HIPCHECK(hipMemcpyAsync(adj->RK, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
-    quad_gram(L, m, rr, shifted_chol(m));
+    hold_matrix(L, m, rr);
     EpiArgs eN = de_epi(EPI_BUG_N);  // N = V1'V0, Sinit = M S0 N'
     eN.S = S;
     eN.ld_s = (int)rcap;
-    cholqr_tail(L, L2, m, rr, V2, true, V, rr, eN, 0, 3);
+    qr(shifted_chol(m), L, L2, m, rr, V2, true, V, eN, 0, 3);
     HIPCHECK(hipMemcpyAsync(adj->RL, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
     quad_galerkin(U2, true, rr);  // U1'AU1, G'U1, W(U1)
     quad_galerkin(V2, false, rr);  // V1'BV1, H'V1, T(V1)
@@ -2941,8 +2967,8 @@ struct lri_ctx {
     QuadStepsArgs KA = quad_steps_args(true, rr, qa->Gb0, qa->hbT0, qa->T0, h);
     KA.store = stK;
     quad_steps(KA, K, work, QuadStepsArgs{}, nullptr, nullptr, nsub);
-    quad_gram(K, n, rr, shifted_chol(n));
-    cholqr_tail(K, K2, n, rr, U2, false, nullptr, 0, de_epi(), 0, 3);  // U1, R1
+    hold_matrix(K, n, rr);
+    qr(shifted_chol(n), K, K2, n, rr, U2, false, nullptr, de_epi(), 0, 3);  // U1, R1
     HIPCHECK(hipMemcpyAsync(adj->RK, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
     // U1's Galerkin data (kept in qa->Ga0, gaT0, W0); S~ from R1; L with its sub-step starts
     quad_galerkin(U2, true, rr);
@@ -2954,8 +2980,8 @@ struct lri_ctx {
     QuadStepsArgs LA = quad_steps_args(false, rr, qa->Ga0, qa->gaT0, qa->W0, h);
     LA.store = stL;
     quad_steps(LA, L, work, QuadStepsArgs{}, nullptr, nullptr, nsub);
-    quad_gram(L, m, rr, shifted_chol(m));
-    cholqr_tail(L, L2, m, rr, V2, true, nullptr, 0, de_epi(), 0, 3);  // V1, R2
+    hold_matrix(L, m, rr);
+    qr(shifted_chol(m), L, L2, m, rr, V2, true, nullptr, de_epi(), 0, 3);  // V1, R2
     HIPCHECK(hipMemcpyAsync(adj->RL, small->Rtot, rsz, hipMemcpyDeviceToDevice, stream));
     // Lbar1: R2 R2bar' = RL Sb1 (adj->Mb), then the QR rule
     timed(LRI_KERNEL_SMALL, [&] { return launch_ksl_adj_small(adj, rr, 0, stream); });
@@ -3462,13 +3488,13 @@ struct lri_ctx {
     const EpiArgs none = de_epi();
     de_galerkin(V, false, rr, de->Gb, de->hbT);  // Bt = V0'BV0
     de_eig(de->Gb, rr, de->Wb, de->beta);
-    de_substep(U, true, rr, S, (int)rcap, 0, de->Wb, de->beta, de->hbT, h, nsub, K, K2, shifted_chol(n));  // K
-    cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 0, 3);                                            // U1, R
+    de_substep(U, true, rr, S, (int)rcap, 0, de->Wb, de->beta, de->hbT, h, nsub, K, K2, true);  // K
+    qr(shifted_chol(n), K, K2, n, rr, U, false, nullptr, none, 0, 3);                                            // U1, R
     de_galerkin(U, true, rr, de->Ga, de->gaT);  // At = U1'AU1
     de_eig(de->Ga, rr, de->Wa, de->alpha);
     de_sstep(rr, rr, small->Rtot, rr, 0, de->Snew, rr, -1.0, h, nsub);  // S~
-    de_substep(V, false, rr, de->Snew, rr, 1, de->Wa, de->alpha, de->gaT, h, nsub, L, L2, shifted_chol(m));  // L
-    cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 2, 3);  // V1, S = R'
+    de_substep(V, false, rr, de->Snew, rr, 1, de->Wa, de->alpha, de->gaT, h, nsub, L, L2, true);  // L
+    qr(shifted_chol(m), L, L2, m, rr, V, true, nullptr, none, 2, 3);  // V1, S = R'
   }
 
   // dual_LT_step! with the DE sub-problems (projector_splitting.jl:52-80,166-189)
@@ -3482,13 +3508,13 @@ struct lri_ctx {
     const EpiArgs none = de_epi();
     de_galerkin(U, true, rr, de->Ga, de->gaT);  // At = U0'AU0
     de_eig(de->Ga, rr, de->Wa, de->alpha);
-    de_substep(V, false, rr, S, (int)rcap, 1, de->Wa, de->alpha, de->gaT, h, nsub, L, L2, shifted_chol(m));  // L
-    cholqr_tail(L, L2, m, rr, V, true, nullptr, 0, none, 0, 3);                                              // V1, R
+    de_substep(V, false, rr, S, (int)rcap, 1, de->Wa, de->alpha, de->gaT, h, nsub, L, L2, true);  // L
+    qr(shifted_chol(m), L, L2, m, rr, V, true, nullptr, none, 0, 3);                                              // V1, R
     de_galerkin(V, false, rr, de->Gb, de->hbT);  // Bt = V1'BV1
     de_eig(de->Gb, rr, de->Wb, de->beta);
     de_sstep(rr, rr, small->Rtot, rr, 1, de->Snew, rr, -1.0, h, nsub);  // S~ from R'
-    de_substep(U, true, rr, de->Snew, rr, 0, de->Wb, de->beta, de->hbT, h, nsub, K, K2, shifted_chol(n));  // K
-    cholqr_tail(K, K2, n, rr, U, false, nullptr, 0, none, 1, 3);  // U1, S = R
+    de_substep(U, true, rr, de->Snew, rr, 0, de->Wb, de->beta, de->hbT, h, nsub, K, K2, true);  // K
+    qr(shifted_chol(n), K, K2, n, rr, U, false, nullptr, none, 1, 3);  // U1, S = R
   }
 
   // unconventional_step! with the DE sub-problems (unconventional.jl:51-79,133-157)
@@ -3518,14 +3544,14 @@ struct lri_ctx {
     const RK4ColArgs Pk = de_prepare(U, true, rr, S, (int)rcap, 0, de->Wb, de->beta, de->hbT, 0, h, nsub, K2);
     const RK4ColArgs Pl = de_prepare(V, false, rr, S, (int)rcap, 1, de->Wa, de->alpha, de->gaT, 1, h, nsub, lscr);
     de_run(Pk, Pl);
-    de_finish(true, rr, de->Wb, K, K2, shifted_chol(n));
+    de_finish_hold(true, rr, de->Wb, K, K2);
     EpiArgs eM = de_epi(EPI_BUG_M);  // M = U1' U0
-    cholqr_tail(K, K2, n, rr, U2, false, U, rr, eM, 0, 3);
-    de_finish(false, rr, de->Wa, L, lscr, shifted_chol(m));
+    qr(shifted_chol(n), K, K2, n, rr, U2, false, U, eM, 0, 3);
+    de_finish_hold(false, rr, de->Wa, L, lscr);
     EpiArgs eN = de_epi(EPI_BUG_N);  // N = V1' V0, Sinit = M S0 N'
     eN.S = S;
     eN.ld_s = (int)rcap;
-    cholqr_tail(L, L2, m, rr, V2, true, V, rr, eN, 0, 3);
+    qr(shifted_chol(m), L, L2, m, rr, V2, true, V, eN, 0, 3);
     de_galerkin(U2, true, rr, de->Ga, de->gaT);   // At = U1'AU1
     de_galerkin(V2, false, rr, de->Gb, de->hbT);  // Bt = V1'BV1
     de_eig2(rr, rr);
@@ -3543,7 +3569,6 @@ struct lri_ctx {
     const int rr = (int)r;
     const int k2 = 2 * rr;
     const double h = dt / (double)nsub;
-    EpiArgs none;
     de_galerkin(V, false, rr, de->Gb, de->hbT);  // Bt = V0'BV0
     de_galerkin(U, true, rr, de->Ga, de->gaT);   // At = U0'AU0
     de_eig2(rr, rr);
@@ -3551,8 +3576,8 @@ struct lri_ctx {
     const RK4ColArgs Pk = de_prepare(U, true, rr, S, (int)rcap, 0, de->Wb, de->beta, de->hbT, 0, h, nsub, K2);
     const RK4ColArgs Pl = de_prepare(V, false, rr, S, (int)rcap, 1, de->Wa, de->alpha, de->gaT, 1, h, nsub, lscr);
     de_run(Pk, Pl);
-    de_finish(true, rr, de->Wb, K, K2, none);
-    de_finish(false, rr, de->Wa, L, lscr, none);
+    rows(de_finish_args(true, rr, de->Wb, K, K2));
+    rows(de_finish_args(false, rr, de->Wa, L, lscr));
     dcopy(Uhat, U, n * rr);
     EpiArgs eM;
     eM.kind = EPI_RA_M;
@@ -3688,6 +3713,7 @@ struct lri_ctx {
     HIPCHECK(hipMemcpy(&f, flags, sizeof(int), hipMemcpyDeviceToHost));
     if (f) HIPCHECK(hipMemset(flags, 0, sizeof(int)));
     if (timing) drain_timing();
+    if (f & FLAG_TIMEOUT) throw Failure{LRI_EHIP, "a device-side wait between workgroups timed out"};
     if (f & FLAG_NONFINITE) return LRI_ENONFINITE;
     if (f & FLAG_BREAKDOWN) return LRI_EBREAKDOWN;
     return LRI_OK;

@@ -207,6 +207,33 @@ struct RowArgs {
 template <typename PT>
 hipError_t launch_rows(RowArgs<PT> A, hipStream_t st);
 
+// A CholeskyQR2 / shifted CholeskyQR3 in one launch (see lri_rowops.hip): form's matrix
+// (written to form.out if set; no stencil, unit signs) = q R, form's packed outputs
+// holding q.  W (n x r) for stilde (as EpiArgs::stilde) or for fin, the epilogue of q' W
+// (EPI_NONE: none).
+template <typename PT>
+struct QrArgs {
+  RowArgs<PT> form;
+  double* q = nullptr;
+  int passes = 2;
+  int64_t shift_rows = 0;                 // first pass
+  int first_error = 1, later_error = 1;   // breakdown_is_error of the first and the later passes
+  double* S = nullptr;                    // S = R (transpose_s: R'), if set
+  int ld_s = 0, transpose_s = 0;
+  int stilde = 0;                         // passes = 2
+  const double* W = nullptr;
+  int64_t ldw = 0;
+  EpiArgs fin;
+  SmallState* small = nullptr;
+  double* gpart = nullptr;
+  int* sync = nullptr;  // two zeroed words, zero again at the end
+  int* flags = nullptr;
+  int tr = 0, blocks = 0;  // filled by the launcher
+};
+bool qr_fits(int64_t rows, int r, int passes);
+template <typename PT>
+hipError_t launch_qr(QrArgs<PT> Q, hipStream_t st);
+
 struct SvdArgs {
   const double* S = nullptr;  // k x k, ld lds
   int lds = 0;

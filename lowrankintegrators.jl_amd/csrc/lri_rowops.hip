@@ -411,149 +411,157 @@ __host__ __device__ inline int epi_scratch_doubles(int kind, int a, int b) {
 // reduction runs in one workgroup; folded into the prologue of the next row
 // kernel, every workgroup computes the factors for itself and workgroup 0
 // stores them).  The Cholesky kinds use C's first a columns as the Gram matrix.
+//
+// The Cholesky kinds.  own_right, own_nd: the factor on the right (LDS) and the first pass's
+// dropped count, for a caller that runs all passes in one launch; nd_out receives this
+// pass's count.
 template <int CK>
-__device__ void run_epilogue(const EpiArgs& E, double* C, int a, int b, double* scr, bool writer = true) {
+__device__ void chol_epilogue(const EpiArgs& E, double* C, int a, double* scr, bool writer,
+                              const double* own_right = nullptr, int own_nd = 0, int* nd_out = nullptr) {
+  const int t = threadIdx.x;
+  SmallState* st = E.small;
+  const int k = a;
+  __shared__ unsigned char dropped[kMaxAug];
+  __shared__ int s_big;
+  __shared__ double s_shift;
+  if (E.kind == EPI_CHOL1 && E.shift_rows > 0) {
+    // shifted CholeskyQR3, first factor: G + s I (Fukaya, Kannan, Nakatsukasa, Yamamoto,
+    // Yanagisawa 2020), with ||G||_2 bounded by trace(G)
+    if (t < 64) {
+      double tr = 0.0;
+      for (int i = t; i < k; i += 64) tr += C[i + i * k];
+      for (int off = 32; off > 0; off >>= 1) tr += __shfl_xor(tr, off);
+      if (t == 0) s_shift = 11.0 * ((double)E.shift_rows * k + (double)k * (k + 1)) * (0.5 * kEps) * tr;
+    }
+    __syncthreads();
+    for (int i = t; i < k; i += blockDim.x) C[i + i * k] += s_shift;
+    __syncthreads();
+  }
+  double* R = scr;
+  double* Rinv = scr + k * k;
+  int nf = 0, nd = 0;
+  // CHOL2/3: the factor on the right of Rtot (R1, or the running Rtot) and
+  // the first pass's dropped count were written by an earlier launch on
+  // this stream; their loads are issued now, ahead of the factorisation
+  // (for CK <= 32; the CK = 64 variant has no registers to spare)
+  constexpr int NQ = CK <= 32 ? (CK * CK) / kThreads : 0;
+  const double* right = own_right ? own_right : E.kind == EPI_CHOL2 ? st->R1 : st->Rtot;
+  double rv[NQ > 0 ? NQ : 1];
+  if (E.kind != EPI_CHOL1) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int e = t + kThreads * q;
+      rv[q] = e < k * k ? right[e] : 0.0;
+    }
+  }
+  const int nd_first = E.kind == EPI_CHOL1 ? 0 : own_right ? own_nd : st->ndropped;
+  // CholeskyQR2's second Gram matrix is I + E with |E| ~ eps cond^2: when
+  // max|E| <= 1e-6 (and the first pass dropped nothing), R = I + F with
+  // F = F1 + F2, F1 = upper(E) (diagonal halved), F2 = upper(-F1'F1)
+  // (diagonal halved), and R^{-1} = I - F + F^2, all exact to O(|E|^3).
+  bool pert = false;
+  if (E.kind != EPI_CHOL1 && nd_first == 0) {
+    if (t == 0) s_big = 0;
+    __syncthreads();
+    double mx = 0.0;
+    for (int e = t; e < k * k; e += blockDim.x) {
+      const int i = e % k, jj = e / k;
+      const double v = C[e] - (i == jj ? 1.0 : 0.0);
+      mx = fmax(mx, isfinite(v) ? fabs(v) : 1e300);
+    }
+    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
+    if ((t & 63) == 0 && mx > 1e-6) atomicOr(&s_big, 1);  // any wave over the bound -> full Cholesky
+    __syncthreads();
+    pert = (s_big == 0);
+  }
+  if (pert) {
+    double* F1 = Rinv;  // scratch: F1, then F1'F1 into R
+    for (int e = t; e < k * k; e += blockDim.x) {
+      const int i = e % k, jj = e / k;
+      const double v = C[e] - (i == jj ? 1.0 : 0.0);
+      F1[e] = i < jj ? v : (i == jj ? 0.5 * v : 0.0);
+    }
+    __syncthreads();
+    small_gemm(F1, 1, F1, 0, R, k);  // R <- F1' F1
+    __syncthreads();
+    for (int e = t; e < k * k; e += blockDim.x) {  // C <- F = F1 + upper(-F1'F1) (diag halved)
+      const int i = e % k, jj = e / k;
+      const double f2 = i < jj ? -R[e] : (i == jj ? -0.5 * R[e] : 0.0);
+      C[e] = F1[e] + f2;
+    }
+    __syncthreads();
+    small_gemm(C, 0, C, 0, Rinv, k);  // Rinv <- F^2
+    __syncthreads();
+    for (int e = t; e < k * k; e += blockDim.x) {
+      const int i = e % k, jj = e / k;
+      const double id = i == jj ? 1.0 : 0.0;
+      R[e] = id + C[e];
+      Rinv[e] = id - C[e] + Rinv[e];
+    }
+    if (t < k) dropped[t] = 0;
+    __syncthreads();
+  } else {
+    nd = chol_inv<CK>(C, R, Rinv, k, dropped, &nf);
+  }
+  if (E.kind == EPI_CHOL1) {
+    if (writer)
+      for (int e = t; e < k * k; e += blockDim.x) {
+        st->R1[e] = R[e];
+        st->R1inv[e] = Rinv[e];
+      }
+  } else {
+    // Rtot = R2 * R1 (CHOL2) or R3 * Rtot (CHOL3) into the third scratch
+    // matrix; the factor on the right was written by an earlier launch on
+    // this stream; C is free now
+    double* Rt = scr + 2 * k * k;
+    if (own_right && !writer) return;  // a one-launch caller's workgroups need R^{-1} only
+    if (writer)
+      for (int e = t; e < k * k; e += blockDim.x) st->R2inv[e] = Rinv[e];
+    if (NQ > 0) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int e = t + kThreads * q;
+        if (e < k * k) C[e] = rv[q];
+      }
+    } else {
+      for (int e = t; e < k * k; e += blockDim.x) C[e] = right[e];
+    }
+    __syncthreads();
+    small_gemm(R, 0, C, 0, Rt, k);
+    __syncthreads();
+    if (writer)
+      for (int e = t; e < k * k; e += blockDim.x) {
+        const int i = e % k, jj = e / k;
+        st->Rtot[e] = Rt[e];
+        if (E.S) E.S[i + jj * E.ld_s] = E.transpose ? Rt[jj + i * k] : Rt[e];
+      }
+    if (E.stilde) {
+      // C = [Q1'Q1 | Q1'W]: U1 = Q1 R2^{-1}, so U1'W = R2^{-T} (Q1'W) and
+      // S~ = Rtot - U1'W; the first k columns of C are free again
+      small_gemm(Rinv, 1, C + k * k, 0, C, k);
+      __syncthreads();
+      if (writer)
+        for (int e = t; e < k * k; e += blockDim.x) {
+          const int i = e % k, jj = e / k;
+          const double v = Rt[e] - C[e];
+          if (E.stilde == 2) st->St[jj + i * k] = v;
+          else st->St[e] = v;
+        }
+    }
+  }
+  if (t == 0 && writer) {
+    if (nf) atomicOr(E.flags, FLAG_NONFINITE);
+    if (nd && E.breakdown_is_error) atomicOr(E.flags, FLAG_BREAKDOWN);
+    if (E.kind == EPI_CHOL1) st->ndropped = nd;
+  }
+  if (t == 0 && nd_out) *nd_out = nd;
+}
+
+// The others (one workgroup).
+__device__ void plain_epilogue(const EpiArgs& E, double* C, int a, int b, double* scr) {
   const int t = threadIdx.x;
   SmallState* st = E.small;
   switch (E.kind) {
-    case EPI_CHOL1:
-    case EPI_CHOL2:
-    case EPI_CHOL3: {
-      const int k = a;
-      __shared__ unsigned char dropped[kMaxAug];
-      __shared__ int s_big;
-      __shared__ double s_shift;
-      if (E.kind == EPI_CHOL1 && E.shift_rows > 0) {
-        // shifted CholeskyQR3, first factor: G + s I (Fukaya, Kannan, Nakatsukasa, Yamamoto,
-        // Yanagisawa 2020), with ||G||_2 bounded by trace(G)
-        if (t < 64) {
-          double tr = 0.0;
-          for (int i = t; i < k; i += 64) tr += C[i + i * k];
-          for (int off = 32; off > 0; off >>= 1) tr += __shfl_xor(tr, off);
-          if (t == 0) s_shift = 11.0 * ((double)E.shift_rows * k + (double)k * (k + 1)) * (0.5 * kEps) * tr;
-        }
-        __syncthreads();
-        for (int i = t; i < k; i += blockDim.x) C[i + i * k] += s_shift;
-        __syncthreads();
-      }
-      double* R = scr;
-      double* Rinv = scr + k * k;
-      int nf = 0, nd = 0;
-      // CHOL2/3: the factor on the right of Rtot (R1, or the running Rtot) and
-      // the first pass's dropped count were written by an earlier launch on
-      // this stream; their loads are issued now, ahead of the factorisation
-      // (for CK <= 32; the CK = 64 variant has no registers to spare)
-      constexpr int NQ = CK <= 32 ? (CK * CK) / kThreads : 0;
-      const double* right = E.kind == EPI_CHOL2 ? st->R1 : st->Rtot;
-      double rv[NQ > 0 ? NQ : 1];
-      if (E.kind != EPI_CHOL1) {
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-          const int e = t + kThreads * q;
-          rv[q] = e < k * k ? right[e] : 0.0;
-        }
-      }
-      const int nd_first = E.kind != EPI_CHOL1 ? st->ndropped : 0;
-      // CholeskyQR2's second Gram matrix is I + E with |E| ~ eps cond^2: when
-      // max|E| <= 1e-6 (and the first pass dropped nothing), R = I + F with
-      // F = F1 + F2, F1 = upper(E) (diagonal halved), F2 = upper(-F1'F1)
-      // (diagonal halved), and R^{-1} = I - F + F^2, all exact to O(|E|^3).
-      bool pert = false;
-      if (E.kind != EPI_CHOL1 && nd_first == 0) {
-        if (t == 0) s_big = 0;
-        __syncthreads();
-        double mx = 0.0;
-        for (int e = t; e < k * k; e += blockDim.x) {
-          const int i = e % k, jj = e / k;
-          const double v = C[e] - (i == jj ? 1.0 : 0.0);
-          mx = fmax(mx, isfinite(v) ? fabs(v) : 1e300);
-        }
-        for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
-        if ((t & 63) == 0 && mx > 1e-6) atomicOr(&s_big, 1);  // any wave over the bound -> full Cholesky
-        __syncthreads();
-        pert = (s_big == 0);
-      }
-      if (pert) {
-        double* F1 = Rinv;  // scratch: F1, then F1'F1 into R
-        for (int e = t; e < k * k; e += blockDim.x) {
-          const int i = e % k, jj = e / k;
-          const double v = C[e] - (i == jj ? 1.0 : 0.0);
-          F1[e] = i < jj ? v : (i == jj ? 0.5 * v : 0.0);
-        }
-        __syncthreads();
-        small_gemm(F1, 1, F1, 0, R, k);  // R <- F1' F1
-        __syncthreads();
-        for (int e = t; e < k * k; e += blockDim.x) {  // C <- F = F1 + upper(-F1'F1) (diag halved)
-          const int i = e % k, jj = e / k;
-          const double f2 = i < jj ? -R[e] : (i == jj ? -0.5 * R[e] : 0.0);
-          C[e] = F1[e] + f2;
-        }
-        __syncthreads();
-        small_gemm(C, 0, C, 0, Rinv, k);  // Rinv <- F^2
-        __syncthreads();
-        for (int e = t; e < k * k; e += blockDim.x) {
-          const int i = e % k, jj = e / k;
-          const double id = i == jj ? 1.0 : 0.0;
-          R[e] = id + C[e];
-          Rinv[e] = id - C[e] + Rinv[e];
-        }
-        if (t < k) dropped[t] = 0;
-        __syncthreads();
-      } else {
-        nd = chol_inv<CK>(C, R, Rinv, k, dropped, &nf);
-      }
-      if (E.kind == EPI_CHOL1) {
-        if (writer)
-          for (int e = t; e < k * k; e += blockDim.x) {
-            st->R1[e] = R[e];
-            st->R1inv[e] = Rinv[e];
-          }
-      } else {
-        // Rtot = R2 * R1 (CHOL2) or R3 * Rtot (CHOL3) into the third scratch
-        // matrix; the factor on the right was written by an earlier launch on
-        // this stream; C is free now
-        double* Rt = scr + 2 * k * k;
-        if (writer)
-          for (int e = t; e < k * k; e += blockDim.x) st->R2inv[e] = Rinv[e];
-        if (NQ > 0) {
-#pragma unroll
-          for (int q = 0; q < NQ; ++q) {
-            const int e = t + kThreads * q;
-            if (e < k * k) C[e] = rv[q];
-          }
-        } else {
-          for (int e = t; e < k * k; e += blockDim.x) C[e] = right[e];
-        }
-        __syncthreads();
-        small_gemm(R, 0, C, 0, Rt, k);
-        __syncthreads();
-        if (writer)
-          for (int e = t; e < k * k; e += blockDim.x) {
-            const int i = e % k, jj = e / k;
-            st->Rtot[e] = Rt[e];
-            if (E.S) E.S[i + jj * E.ld_s] = E.transpose ? Rt[jj + i * k] : Rt[e];
-          }
-        if (E.stilde) {
-          // C = [Q1'Q1 | Q1'W]: U1 = Q1 R2^{-1}, so U1'W = R2^{-T} (Q1'W) and
-          // S~ = Rtot - U1'W; the first k columns of C are free again
-          small_gemm(Rinv, 1, C + k * k, 0, C, k);
-          __syncthreads();
-          if (writer)
-            for (int e = t; e < k * k; e += blockDim.x) {
-              const int i = e % k, jj = e / k;
-              const double v = Rt[e] - C[e];
-              if (E.stilde == 2) st->St[jj + i * k] = v;
-              else st->St[e] = v;
-            }
-        }
-      }
-      if (t == 0 && writer) {
-        if (nf) atomicOr(E.flags, FLAG_NONFINITE);
-        if (nd && E.breakdown_is_error) atomicOr(E.flags, FLAG_BREAKDOWN);
-        if (E.kind == EPI_CHOL1) st->ndropped = nd;
-      }
-      break;
-    }
     case EPI_STILDE: {
       const int k = a;
       for (int e = t; e < k * k; e += blockDim.x) {
@@ -661,6 +669,12 @@ __device__ void run_epilogue(const EpiArgs& E, double* C, int a, int b, double* 
     default:
       break;
   }
+}
+
+template <int CK>
+__device__ void run_epilogue(const EpiArgs& E, double* C, int a, int b, double* scr, bool writer = true) {
+  if (E.kind == EPI_CHOL1 || E.kind == EPI_CHOL2 || E.kind == EPI_CHOL3) chol_epilogue<CK>(E, C, a, scr, writer);
+  else plain_epilogue(E, C, a, b, scr);
 }
 
 // Partial sums of the per-workgroup reductions: workgroup b of k_reduce sums
@@ -1156,6 +1170,520 @@ hipError_t launch_rows(RowArgs<PT> A, hipStream_t st) {
 
 template hipError_t launch_rows<double>(RowArgs<double>, hipStream_t);
 template hipError_t launch_rows<float>(RowArgs<float>, hipStream_t);
+
+// ----------------------------------------------------------------------------
+// A whole CholeskyQR2 (or shifted CholeskyQR3) of an n x r matrix, r <= 32, in one
+// launch: the formation of the matrix (as k_rows: split partials, a base, X op(Y)),
+// the Gram matrices and their factors, the applications of R^{-1}, the packed
+// copy and the reduction against W.  At these sizes every step is far below the
+// cost of a launch (4 to 5 us each, and each kernel starts by fetching what the one
+// before wrote): the chain rows - reduce - rows - reduce - rows took 52 us for 256 x 8 and
+// 68 us for 2000 x 21, this launch 27 and 50 us; shifted CholeskyQR3 of 4096 x 32 went
+// from 113 to 87 us, of 1000 x 15 from 84 to 38 us (8 us of each pass are the serial
+// 32-pivot Cholesky, 4 us at r <= 16).
+//
+// G <= 64 workgroups keep their rows in LDS from start to end.  A Gram matrix is
+// summed over them through memory: every workgroup writes its part with
+// write-through stores, waits for them, adds to a counter and waits until all
+// have (2 us measured); then each sums all parts in workgroup order (the same bits
+// everywhere, whatever the timing) and factors redundantly, as the prologues of
+// k_rows do.  One workgroup more, without rows, forms what the step's later kernels
+// need (Rtot, S~, the reduction against W) while the others apply R^{-1} and store.
+// The workgroups take one CU each and are resident at once on an idle device; with
+// other kernels running they become so when those end.  A wait is bounded all
+// the same (kQrSpins polls, then FLAG_TIMEOUT and the kernel runs to its end).  The last
+// workgroup out resets the counters, so that a captured launch can be replayed.  A
+// matrix that one workgroup's LDS holds is done by one alone.
+// ----------------------------------------------------------------------------
+
+constexpr int kQrThreads = kThreads, kQrMaxBlocks = 64, kQrDirect = 20, kQrSlots = 4, kQrSpins = 1 << 21;
+
+struct QrShape {
+  int blocks, tr;  // workgroups with rows, rows of each (a multiple of 16)
+};
+// CK = 16 or 32 padded columns
+__host__ __device__ inline int qr_max_tile(int ck) { return ck == 16 ? 768 : 256; }
+__host__ __device__ inline QrShape qr_shape(int64_t rows, int ck) {
+  const int alone = ck == 16 ? 512 : 256, tile = ck == 16 ? 256 : 128;
+  if (rows <= alone) return {1, (int)((rows + 15) / 16 * 16)};
+  int tr = tile;
+  while ((rows + tr - 1) / tr > kQrMaxBlocks) tr += 16;
+  return {(int)((rows + tr - 1) / tr), tr};
+}
+// Two passes over more than 6144 rows stay with the separate kernels at r > 16: exchanging the
+// parts of 48 workgroups and more costs what the launches did (16384 x 32: 83 us against
+// 85; 2000 x 21: 50 against 68), three passes gain at every size (4096 x 32: 87 against 113).
+bool qr_fits(int64_t rows, int r, int passes) {
+  if (r < 1 || r > 32) return false;
+  const int ck = r <= 16 ? 16 : 32;
+  if (passes == 2 && ck == 32 && rows > 6144) return false;
+  return rows <= (int64_t)kQrMaxBlocks * qr_max_tile(ck);
+}
+__host__ __device__ inline int qr_lds_doubles(int tr, int ck) { return tr * (ck + 1) + 4 * ck * (ck + 1) + (2 + 3 + 1) * ck * ck; }
+
+template <typename PT, int CK>
+__global__ __launch_bounds__(kQrThreads) void k_qr(QrArgs<PT> Q) {
+  extern __shared__ double lds[];
+  __shared__ int s_nd;
+  constexpr int LD = CK + 1, NT = CK / 16, KS = CK / 4, NW = kQrThreads / 64;
+  const RowArgs<PT>& A = Q.form;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 15, lk = lane >> 4;
+  const int r = A.r_out, tr = Q.tr, G = Q.blocks, bid = blockIdx.x;
+  const bool rows_wg = bid < G;             // has rows
+  const bool scribe = G == 1 || bid == G;   // writes the small results
+  const int64_t row0 = (int64_t)bid * tr;
+  const int nrows = rows_wg ? (int)min((int64_t)tr, A.rows - row0) : 0;
+  double* kt = lds;                 // the tile, kt[row * LD + column], zero beyond the data
+  double* red = kt + tr * LD;       // a wave's partial reductions [i + LD j]; operands [k * LD + n]
+  double* C = red + NW * CK * LD;   // r x 2r
+  double* scr = C + 2 * CK * CK;    // R, R^{-1}, Rtot
+  double* Rr = scr + 3 * CK * CK;   // the factor on the right of the next pass
+  const int strips = rows_wg ? tr / 16 : 0;  // of 16 rows, wave w taking w, w + NW, ...
+
+  // rows of X (n x r, ld) in operand layout for four of the wave's strips from number si on:
+  // lane lr = row, 4 j + lk = column
+  auto load_x = [&](double (&x)[4][KS], int si) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int lrow = (wave + NW * (si + q)) * 16 + lr;
+#pragma unroll
+      for (int j = 0; j < KS; ++j) {
+        const int d = 4 * j + lk;
+        x[q][j] = lrow < nrows && d < r ? A.X[row0 + lrow + d * A.ldx] : 0.0;
+      }
+    }
+  };
+  // rows of W for the reduction: lane lr = column, 4 j + lk = row
+  auto load_w = [&](double (&w)[4][4][NT], int si) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const int lrow = (wave + NW * (si + q)) * 16 + 4 * j + lk;
+          w[q][j][n] = lrow < nrows && 16 * n + lr < r ? Q.W[row0 + lrow + (16 * n + lr) * Q.ldw] : 0.0;
+        }
+  };
+
+  // ---- the matrix: split partials + base + X op(Y)
+  if (rows_wg) {
+    double x[4][KS];
+    if (A.X) {
+      load_x(x, 0);
+      for (int e = t; e < CK * CK; e += kQrThreads) {
+        const int d = e % CK, c = e / CK;  // red[d * LD + c] = op(Y)(d, c)
+        red[d * LD + c] = d < r && c < r ? (A.transY ? A.Y[c + d * A.ldy] : A.Y[d + c * A.ldy]) : 0.0;
+      }
+    }
+    constexpr int U = CK / NW, B = 2;  // columns of a wave, blocks of 64 rows, loaded together
+    const int64_t ss = (int64_t)A.rb * A.rows;
+    for (int l0 = lane; l0 < tr; l0 += 64 * B) {
+      double v[B][U];
+      int64_t i[B];
+#pragma unroll
+      for (int k = 0; k < B; ++k) {
+        i[k] = row0 + (l0 + 64 * k < nrows ? l0 + 64 * k : 0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[k][u] = 0.0;
+      }
+      if (A.parts) {
+        for (int sp = 0; sp < A.nsplit; sp += 4) {
+          PT w[B][U][4];
+#pragma unroll
+          for (int k = 0; k < B; ++k)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                w[k][u][q] = A.parts[min(sp + q, A.nsplit - 1) * ss + (int64_t)min(wave + NW * u, r - 1) * A.rows + i[k]];
+#pragma unroll
+          for (int k = 0; k < B; ++k)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                if (sp + q < A.nsplit) v[k][u] += (double)w[k][u][q];
+        }
+      }
+      if (A.base) {
+        double w[B][U];
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+#pragma unroll
+          for (int u = 0; u < U; ++u) w[k][u] = A.base[i[k] + (int64_t)min(wave + NW * u, r - 1) * A.ld_base];
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[k][u] += w[k][u];
+      }
+#pragma unroll
+      for (int k = 0; k < B; ++k)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int c = wave + NW * u, lrow = l0 + 64 * k;
+          const bool ok = c < r && lrow < nrows;
+          if (A.sum_out && ok) A.sum_out[i[k] + c * A.ld_sum] = v[k][u];
+          if (lrow < tr) kt[lrow * LD + c] = ok ? v[k][u] : 0.0;
+        }
+    }
+    __syncthreads();
+    if (A.X) {
+      for (int si = 0; wave + NW * si < strips; si += 4) {
+        if (si) load_x(x, si);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int s = wave + NW * (si + q);
+          if (s < strips)
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            f64x4_t acc;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[u] = kt[(s * 16 + 4 * u + lk) * LD + 16 * n + lr];
+#pragma unroll
+            for (int j = 0; j < KS; ++j)
+              acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[q][j], red[(4 * j + lk) * LD + 16 * n + lr], acc, 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) kt[(s * 16 + 4 * u + lk) * LD + 16 * n + lr] = acc[u];
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+  auto copy_out = [&](double* dst, int64_t ld) {
+    for (int lrow = lane; lrow < nrows; lrow += 64)
+      for (int c = wave; c < r; c += NW) dst[row0 + lrow + c * ld] = kt[lrow * LD + c];
+  };
+  if (A.out) copy_out(A.out, A.ldo);
+
+  int arrived = 0;  // reductions over the workgroups so far
+  // Stores this workgroup's part (r x r) of a reduction, summed over the waves: into C + at
+  // if there is one workgroup, else into its place of `slot`.  sym: only the blocks
+  // on and above the diagonal were formed.
+  auto store_part = [&](int at, int slot, bool sym) {
+    __syncthreads();
+    double* gp = Q.gpart + ((int64_t)slot * G + bid) * r * r;
+    for (int e = t; e < r * r; e += kQrThreads) {
+      int i = e % r, j = e / r;
+      if (sym && (i >> 4) > (j >> 4)) {
+        const int x = i;
+        i = j;
+        j = x;
+      }
+      const int o = i + LD * j;
+      double v = red[o];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) v += red[w * CK * LD + o];
+      if (G == 1) C[at + e] = v;
+      else __hip_atomic_store(gp + e, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+  };
+  auto to_red = [&](int m, int n, const f64x4_t& acc) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) red[wave * CK * LD + 16 * m + 4 * u + lk + LD * (16 * n + lr)] = acc[u];
+  };
+  auto gram = [&](int slot) {  // tile' tile
+    f64x4_t acc[NT][NT];
+#pragma unroll
+    for (int m = 0; m < NT; ++m)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[m][n] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+    for (int s = wave; s < strips; s += NW) {
+      double a[4][NT];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) a[j][n] = kt[(s * 16 + 4 * j + lk) * LD + 16 * n + lr];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+          for (int n = m; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j][m], a[j][n], acc[m][n], 0, 0, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < NT; ++m)
+#pragma unroll
+      for (int n = m; n < NT; ++n) to_red(m, n, acc[m][n]);
+    store_part(0, slot, true);
+  };
+  auto cross = [&](double (&w)[4][4][NT], int at, int slot) {  // tile' W; w: load_w(w, 0)
+    f64x4_t acc[NT][NT];
+#pragma unroll
+    for (int m = 0; m < NT; ++m)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[m][n] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+    for (int si = 0; wave + NW * si < strips; si += 4) {
+      if (si) load_w(w, si);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int s = wave + NW * (si + q);
+        if (s < strips)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int m = 0; m < NT; ++m) {
+            const double a = kt[(s * 16 + 4 * j + lk) * LD + 16 * m + lr];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, w[q][j][n], acc[m][n], 0, 0, 0);
+          }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < NT; ++m)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) to_red(m, n, acc[m][n]);
+    store_part(at, slot, false);
+  };
+  // the stores of this workgroup's parts are done; all workgroups' are when wait returns
+  auto arrive = [&]() {
+    if (G == 1) return;
+    ++arrived;
+    if (!rows_wg) return;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (t == 0) __hip_atomic_fetch_add(Q.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto wait = [&]() {
+    if (G == 1) return;
+    if (t == 0) {
+      int n = 0;
+      while (__hip_atomic_load(Q.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < arrived * G && ++n < kQrSpins)
+        __builtin_amdgcn_s_sleep(1);
+      if (n >= kQrSpins) atomicOr(Q.flags, FLAG_TIMEOUT);
+    }
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  };
+  // C + at <- the sum of all workgroups' parts, G <= kQrDirect: every workgroup adds them up
+  auto sum = [&](int at, int slot) {
+    const double* gp = Q.gpart + (int64_t)slot * G * r * r;
+    constexpr int E = CK * CK / kQrThreads;  // entries of a thread
+    double s[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) s[q] = 0.0;
+    for (int g = 0; g < G; g += 8) {  // 8 workgroups' entries in flight together
+      double v[8][E];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int q = 0; q < E; ++q)
+          v[u][q] = gp[(int64_t)min(g + u, G - 1) * r * r + min(t + kQrThreads * q, r * r - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int q = 0; q < E; ++q) s[q] += g + u < G ? v[u][q] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < E; ++q)
+      if (t + kQrThreads * q < r * r) C[at + t + kQrThreads * q] = s[q];
+    __syncthreads();
+  };
+  // above that (the parts are 8 KB each at r = 32, and reading 64 of them takes one CU
+  // 11 us) a workgroup adds up its share of the entries, thread (entry, quarter) in
+  // workgroup order, and the sums are exchanged like the parts
+  auto share = [&](int slot, int nslots) {
+    const int n = nslots * r * r, len = (n + G - 1) / G;
+    const double* gp = Q.gpart + (int64_t)slot * G * r * r;
+    double* gs = Q.gpart + (int64_t)(kQrSlots + slot) * G * r * r;
+    const int qt = t >> 6;
+    for (int x0 = 0; x0 < len; x0 += 64) {  // once, or twice for two parts of r > 25 and G < 32
+      const int x = bid * len + x0 + (t & 63);
+      const bool mine = rows_wg && x0 + (t & 63) < len && x < n;
+      double s = 0.0;
+      if (mine) {
+        const double* p = gp + (int64_t)(x / (r * r)) * G * r * r + x % (r * r);
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = p[(int64_t)min(qt * 16 + u, G - 1) * r * r];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += qt * 16 + u < G ? v[u] : 0.0;
+      }
+      red[t] = s;
+      __syncthreads();
+      if (mine && qt == 0)
+        __hip_atomic_store(gs + x, ((red[t] + red[64 + t]) + red[128 + t]) + red[192 + t], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+    }
+    arrive();
+    wait();
+    for (int e = t; e < (scribe ? n : r * r); e += kQrThreads) C[e] = gs[e];
+    __syncthreads();
+  };
+  // C <- [the reduction of slot | that of slot + 1 (scribe only)] over all workgroups
+  auto total = [&](int slot, int nslots) {
+    if (G == 1) return;
+    arrive();
+    wait();
+    if (G > kQrDirect) {
+      share(slot, nslots);
+    } else {
+      sum(0, slot);
+      if (nslots > 1 && scribe) sum(r * r, slot + 1);
+    }
+  };
+  // tile <- tile * R^{-1}
+  auto apply = [&]() {
+    const double* Ri = scr + r * r;
+    for (int e = t; e < CK * CK; e += kQrThreads) {
+      const int d = e % CK, c = e / CK;
+      red[d * LD + c] = d < r && c < r ? Ri[d + c * r] : 0.0;
+    }
+    __syncthreads();
+    double b[NT][KS];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int j = 0; j < KS; ++j) b[n][j] = red[(4 * j + lk) * LD + 16 * n + lr];
+    for (int s = wave; s < strips; s += NW) {
+      double a[KS];
+#pragma unroll
+      for (int j = 0; j < KS; ++j) a[j] = kt[(s * 16 + lr) * LD + 4 * j + lk];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        f64x4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < KS; ++j) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j], b[n][j], acc, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) kt[(s * 16 + 4 * u + lk) * LD + 16 * n + lr] = acc[u];
+      }
+    }
+    __syncthreads();
+  };
+
+  int slot = 0, nd = 0;
+  for (int pass = 0; pass < Q.passes; ++pass) {
+    // by value, from scalars: a reference into the argument segment makes the Cholesky spill
+    EpiArgs E;
+    E.kind = pass == 0 ? EPI_CHOL1 : pass == 1 ? EPI_CHOL2 : EPI_CHOL3;
+    E.breakdown_is_error = pass == 0 ? Q.first_error : Q.later_error;
+    E.small = Q.small;
+    E.flags = Q.flags;
+    E.shift_rows = pass == 0 ? Q.shift_rows : 0;
+    E.S = pass == Q.passes - 1 ? Q.S : nullptr;
+    E.ld_s = Q.ld_s;
+    E.transpose = Q.transpose_s;
+    E.stilde = pass == 1 ? Q.stilde : 0;
+    const bool with_w = E.stilde != 0;  // C = tile' [tile | W]
+    if (rows_wg) {
+      if (with_w) {
+        double wv[4][4][NT];
+        load_w(wv, 0);
+        gram(slot);
+        cross(wv, r * r, slot + 1);
+      } else {
+        gram(slot);
+      }
+    }
+    total(slot, with_w ? 2 : 1);
+    slot += with_w ? 2 : 1;
+    chol_epilogue<CK>(E, C, r, scr, scribe, pass ? Rr : nullptr, nd, &s_nd);
+    __syncthreads();
+    if (pass == 0) nd = s_nd;
+    if (scribe)  // only Rtot needs it
+      for (int e = t; e < r * r; e += kQrThreads) Rr[e] = scr[(pass ? 2 * r * r : 0) + e];
+    if (rows_wg) apply();
+    else __syncthreads();
+  }
+  // ---- Q, the reduction against W and the packed copy
+  if (rows_wg) {
+    if (Q.fin.kind != EPI_NONE) {
+      double wv[4][4][NT];
+      load_w(wv, 0);
+      copy_out(Q.q, A.rows);
+      cross(wv, 0, slot);
+    } else {
+      copy_out(Q.q, A.rows);
+    }
+    if (A.pk_f64) {
+      for (int e = t; e < nrows * A.pk_cols; e += kQrThreads) {
+        const int c = e % A.pk_cols, lrow = e / A.pk_cols;
+        A.pk_f64[(row0 + lrow) * A.pk_cols + c] = c < r ? kt[lrow * LD + c] : 0.0;
+      }
+    } else if (A.pk_f32 || A.pk_hi) {
+      // eight consecutive rows of a column lie together in every layout but pass N's FP32 one
+      for (int c = wave; c < A.pk_cols; c += NW)
+        for (int g8 = lane; g8 * 8 < nrows; g8 += 64) {
+          float v[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) v[u] = c < r ? (float)kt[(g8 * 8 + u) * LD + c] : 0.0f;
+          const int64_t i = row0 + g8 * 8;
+          const bool whole = g8 * 8 + 8 <= nrows;
+          if (A.pk_f32) {
+            if (A.pk_layout == 1 && whole) {
+              f32x4_t* d = reinterpret_cast<f32x4_t*>(A.pk_f32 + pk_f32_offset(1, i, c, A.pk_cols));
+              d[0] = f32x4_t{v[0], v[1], v[2], v[3]};
+              d[1] = f32x4_t{v[4], v[5], v[6], v[7]};
+            } else {
+#pragma unroll
+              for (int u = 0; u < 8; ++u)
+                if (g8 * 8 + u < nrows) A.pk_f32[pk_f32_offset(A.pk_layout, i + u, c, A.pk_cols)] = v[u];
+            }
+          }
+          if (A.pk_hi) {
+            uint32_t hi[8], lo[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) split_bf16(v[u], hi[u], lo[u]);
+            const int64_t off = pk_offset(A.pk_layout, i, c, A.pk_cols);
+            if (whole) {
+              *reinterpret_cast<u32x4_t*>(A.pk_hi + off) = u32x4_t{hi[0] | hi[1] << 16, hi[2] | hi[3] << 16,
+                                                                    hi[4] | hi[5] << 16, hi[6] | hi[7] << 16};
+              *reinterpret_cast<u32x4_t*>(A.pk_lo + off) = u32x4_t{lo[0] | lo[1] << 16, lo[2] | lo[3] << 16,
+                                                                    lo[4] | lo[5] << 16, lo[6] | lo[7] << 16};
+            } else {
+#pragma unroll
+              for (int u = 0; u < 8; ++u)
+                if (g8 * 8 + u < nrows) {
+                  A.pk_hi[off + u] = (uint16_t)hi[u];
+                  A.pk_lo[off + u] = (uint16_t)lo[u];
+                }
+            }
+          }
+        }
+    }
+  }
+  if (Q.fin.kind != EPI_NONE) {
+    arrive();
+    if (scribe) {
+      wait();
+      if (G > 1) sum(0, slot);
+      EpiArgs F = Q.fin;
+      plain_epilogue(F, C, r, r, scr);
+    }
+  }
+  if (G > 1) {
+    __syncthreads();
+    if (t == 0 &&
+        __hip_atomic_fetch_add(Q.sync + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == G) {
+      // G workgroups and the scribe are past their last wait
+      __hip_atomic_store(Q.sync, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(Q.sync + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+template <typename PT>
+hipError_t launch_qr(QrArgs<PT> Q, hipStream_t st) {
+  const int r = Q.form.r_out;
+  if (!qr_fits(Q.form.rows, r, Q.passes) || Q.form.rows < 1 || (Q.passes != 2 && Q.passes != 3) || !Q.q || !Q.gpart || !Q.sync ||
+      !Q.flags || (Q.form.X && (Q.form.r_in != r || !Q.form.Y)) || (Q.fin.kind != EPI_NONE && !Q.W) ||
+      Q.form.st_d || Q.form.xy_sign != 1.0 || Q.form.base_sign != 1.0)
+    return hipErrorInvalidValue;
+  const int ck = r <= 16 ? 16 : 32;
+  const QrShape s = qr_shape(Q.form.rows, ck);
+  Q.tr = s.tr;
+  Q.blocks = s.blocks;
+  const size_t lds = sizeof(double) * qr_lds_doubles(s.tr, ck);
+  const dim3 g(s.blocks > 1 ? s.blocks + 1 : 1), b(kQrThreads);
+  if (ck == 16) hipLaunchKernelGGL((k_qr<PT, 16>), g, b, lds, st, Q);
+  else hipLaunchKernelGGL((k_qr<PT, 32>), g, b, lds, st, Q);
+  return hipGetLastError();
+}
+template hipError_t launch_qr<double>(QrArgs<double>, hipStream_t);
+template hipError_t launch_qr<float>(QrArgs<float>, hipStream_t);
 
 // ----------------------------------------------------------------------------
 // one-sided (Hestenes) Jacobi SVD of a k x k FP64 matrix, k <= 128, in one
