@@ -4001,8 +4001,7 @@ struct MergedPhase {
       case KID_ROWS_F:
       case KID_REDUCE:
       case KID_EPILOGUE:
-      case KID_JACOBI_WAVE:
-      case KID_JACOBI_WG:
+      case KID_JACOBI:
         HIPCHECK(launch_rowops_batched(ln.kid, ln.variant, pool, start, ln.count, ln.total, ln.block, ln.lds, st));
         break;
       default:

@@ -26,8 +26,7 @@ enum KernelId : int {
   KID_ROWS_F,       // k_rows<float, NRB, 0>; variant = NRB
   KID_REDUCE,       // k_reduce
   KID_EPILOGUE,     // k_epilogue<CK>; variant = CK
-  KID_JACOBI_WAVE,  // k_jacobi_wave (two decompositions per record)
-  KID_JACOBI_WG,    // k_jacobi_svd
+  KID_JACOBI,       // k_jacobi_svd (two decompositions per record)
   KID_SYM_EIG,      // k_sym_eig<kP> (one or two decompositions per record); variant = kP
   KID_SHIFT,        // k_shift_sym
   KID_UNSHIFT,      // k_unshift

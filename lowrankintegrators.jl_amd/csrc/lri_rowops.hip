@@ -1689,55 +1689,25 @@ template hipError_t launch_qr<float>(QrArgs<float>, hipStream_t);
 // one-sided (Hestenes) Jacobi SVD of a k x k FP64 matrix, k <= 128, in one
 // workgroup, then the truncation rank (rank_adaptive_unconventional.jl:222-223)
 // r1 = min{rho >= 1 : sqrt(sum_{j >= rho} sigma_j^2) <= tol}, clipped to rmax.
-// Pairs are processed in round-robin (circle-method) order, npairs at a time.
+// Pairs are processed in round-robin (circle-method) order, all at a time.
+//
+// QR preconditioning (Drmac and Veselic, "New fast and accurate Jacobi SVD
+// algorithm", SIAM J. Matrix Anal. Appl. 29, 2008): with S = Q R, the sweeps run on
+// R' instead of S.  Its columns are much closer to orthogonal than those of a
+// graded S, so the sweeps to convergence drop from 15-30 to 6-11 at k = 16..64.
+// With R' J = W (J the accumulated rotations, W = Ur Sigma), S = (Q J) Sigma Ur': the
+// left singular vectors are Q J and the right ones the normalised columns of W.
+//
+// What bounds it is the serial chain of a round: the pair's columns from LDS, three
+// dot products, the rotation's square roots, the columns back, a barrier.  Eight
+// lanes hold a pair (k <= 8 R: R rows of both columns a lane), so the whole of A
+// is one wave per SIMD up to k = 64; the rotations of V, on which the next round does
+// not wait, are applied by as many waves more, one round later.  In the QR and in Q J
+// eight lanes keep one column in registers.  A k = 40 decomposition takes 181 us; with 16
+// lanes a pair in runs over LDS, V on the same lanes and a barrier after every step it
+// took 440.  64 merged members: 309 us up to k = 64 and 531 up to 80 (V in LDS up to 96),
+// where they took 277 (k <= 32 only, one wave each) and 956.
 // ----------------------------------------------------------------------------
-
-// Singular values (column norms of the rotated A, k x ke, ld lda), the sorted
-// outputs U = A / sigma and V, and the truncation rank; nthr threads take part.
-// pre: the sweeps ran on R' of S = Q R and Vm holds Q J, so U = Vm and V = A / sigma.
-__device__ void jacobi_finish(const SvdArgs& P, const double* A, int lda, const double* Vm, int ldv, double* sig,
-                              int nthr, bool pre = false) {
-  const int k = P.k;
-  const int ke = (k + 1) & ~1;
-  const int t = threadIdx.x;
-  for (int j = t; j < ke; j += nthr) {
-    double s = 0.0;
-    if (j < k)
-      for (int i = 0; i < k; ++i) s += A[i + j * lda] * A[i + j * lda];
-    sig[j] = (j < k) ? sqrt(s) : -1.0;
-  }
-  __syncthreads();
-  for (int j = t; j < k; j += nthr) {
-    int pos = 0;
-    for (int l = 0; l < k; ++l) pos += (sig[l] > sig[j]) || (sig[l] == sig[j] && l < j);
-    P.sigma[pos] = sig[j];
-    const double inv = sig[j] > 0.0 ? 1.0 / sig[j] : 0.0;
-    double* Ua = pre ? P.V : P.U;  // the normalised columns of A
-    double* Uv = pre ? P.U : P.V;  // the accumulated rotations
-    for (int i = 0; i < k; ++i) {
-      Ua[i + pos * k] = A[i + j * lda] * inv;
-      Uv[i + pos * k] = Vm[i + j * ldv];
-    }
-  }
-  __syncthreads();
-  if (t == 0) {
-    // P.sigma holds the sorted values (written above by this workgroup)
-    double tail = 0.0;
-    int rho = k;
-    for (int j = k - 1; j >= 1; --j) {
-      double nt = tail + P.sigma[j] * P.sigma[j];
-      if (sqrt(nt) <= P.tol) {
-        tail = nt;
-        rho = j;
-      } else {
-        break;
-      }
-    }
-    if (rho > P.rmax) rho = (int)P.rmax;
-    if (rho < 1) rho = 1;
-    *P.r_out = rho;
-  }
-}
 
 // x from lane (lane ^ m) of its row of 16 for the DPP patterns used below
 template <int CTRL>
@@ -1748,300 +1718,278 @@ __device__ __forceinline__ double dpp_f64(double x) {
   return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
 }
 
-// Sum over aligned groups of G lanes (G a power of two), left in every lane of
-// the group.  Quad swaps (quad_perm [1,0,3,2] and [2,3,0,1]) make every quad
-// uniform; the half-row mirror (lane i <- 7 - i) then pairs the two quads of
-// an 8-lane group and the row mirror (i <- 15 - i) the two halves of a row.
-template <int G>
-__device__ __forceinline__ double group_sum(double x) {
-  if (G >= 2) x += dpp_f64<0xB1>(x);
-  if (G >= 4) x += dpp_f64<0x4E>(x);
-  if (G >= 8) x += dpp_f64<0x141>(x);
-  if (G >= 16) x += dpp_f64<0x140>(x);
-  if (G >= 32) x += __shfl_xor(x, 16, 32);
-  if (G >= 64) x += __shfl_xor(x, 32, 64);
+// Sum over aligned groups of 8 lanes, left in every lane of the group.  Quad swaps
+// (quad_perm [1,0,3,2] and [2,3,0,1]) make every quad uniform; the half-row mirror
+// (lane i <- 7 - i) then pairs the two quads.
+__device__ __forceinline__ double group_sum8(double x) {
+  x += dpp_f64<0xB1>(x);
+  x += dpp_f64<0x4E>(x);
+  x += dpp_f64<0x141>(x);
   return x;
 }
 
-// group_sum for a group size known only at run time (uniform across the workgroup)
-__device__ __forceinline__ double group_sum_rt(double x, int g) {
-  switch (g) {
-    case 1: return x;
-    case 2: return group_sum<2>(x);
-    case 4: return group_sum<4>(x);
-    case 8: return group_sum<8>(x);
-    case 16: return group_sum<16>(x);
-    case 32: return group_sum<32>(x);
-    default: return group_sum<64>(x);
-  }
+// LDS doubles for k <= 8 R.  Column pitches in LDS are odd multiples of 8: neighbouring
+// groups' columns then start 8 doubles (16 banks) apart.
+constexpr int jacobi_lds_doubles(int R) {
+  const int n = 8 * R, ld = n + 8;
+  return (R > 12 ? 1 : 2) * n * ld + 5 * n + 2;
 }
 
-// QR preconditioning of the one-sided Jacobi SVD (Drmac and Veselic, "New
-// fast and accurate Jacobi SVD algorithm", SIAM J. Matrix Anal. Appl. 29,
-// 2008): with S = Q R, the sweeps run on R' instead of S.  Its columns are
-// much closer to orthogonal than those of a graded S, so the sweeps to
-// convergence drop from 15-30 to 6-11 at k = 16..64.  With R' J = W (J the
-// accumulated rotations, W = Ur Sigma), S = (Q J) Sigma Ur': the left
-// singular vectors are Q J and the right ones the normalised columns of W.
-//
-// Householder QR of A (k x k, ld lda), k <= 128, nt threads (a multiple of
-// 64): reflector j (H_j = I - tau_j v v', v_j = 1, as LAPACK's dlarfg) in
-// column j of H (k x k, ld k), tau_j in tau; on return A holds R' (lower
-// triangular).  Wave 0 forms each reflector (rows lane and lane + 64);
-// nt / 64 (k <= 64) or nt / 128 threads per column apply it.  A, H and tau may
-// be in LDS or in global memory (the workgroup barriers order both).
-__device__ void jacobi_qr_precondition(double* A, int lda, int k, double* H, double* tau, int nt) {
-  __shared__ double s_hv[2];  // beta (the new diagonal), tau of the current reflector
+// 64 R threads (others leave at once).  R = 16: V in P.work, where the reflectors wait too
+// (the others keep theirs in registers).
+template <int R>
+__device__ void jacobi_body(const SvdArgs P, double* lds) {
+  constexpr int N = 8 * R, LD = N + 8, LV = R > 12 ? N : LD;
+  const int k = P.k, ke = (k + 1) & ~1;
   const int t = threadIdx.x;
-  const int cap = k > 64 ? 128 : 64;
-  const int gq = nt / cap;  // threads per column
-  const int c = t / gq, ln = t % gq;
-  for (int j = 0; j < k; ++j) {
-    if (t < 64) {
-      const int i0 = t, i1 = t + 64;
-      const double x0 = i0 < k ? A[i0 + j * lda] : 0.0;
-      const double x1 = i1 < k ? A[i1 + j * lda] : 0.0;
-      const double a = j < 64 ? readlane_f64(x0, j) : readlane_f64(x1, j - 64);
-      double s2 = (i0 > j && i0 < k ? x0 * x0 : 0.0) + (i1 > j && i1 < k ? x1 * x1 : 0.0);
-      s2 = group_sum<64>(s2);
-      double beta = a, tj = 0.0, scale = 0.0;
-      if (s2 > 0.0) {
-        beta = -copysign(sqrt(__builtin_fma(a, a, s2)), a);
-        tj = (beta - a) / beta;
-        scale = 1.0 / (a - beta);
-      }
-      if (i0 < k) H[i0 + j * k] = i0 == j ? 1.0 : (i0 > j ? x0 * scale : 0.0);
-      if (i1 < k) H[i1 + j * k] = i1 == j ? 1.0 : (i1 > j ? x1 * scale : 0.0);
-      if (t == 0) {
-        s_hv[0] = beta;
-        s_hv[1] = tj;
-        tau[j] = tj;
-      }
+  if (t >= 64 * R) return;
+  double* A = lds;             // N x N, ld LD
+  double* tau = A + N * LD;
+  double* sig = tau + N;
+  double* sorted = sig + N;
+  double2* cs = reinterpret_cast<double2*>(sorted + N);  // rotations of a round (cos, sin), twice N / 2
+  int* s_rot = reinterpret_cast<int*>(cs + N);           // a rotation in sweep w: s_rot[w % 3]
+  double* Vm = R > 12 ? P.work : sorted + 3 * N + 2;     // N x N, ld LV
+  double* H = A;  // the reflectors, ld LD, while A's columns are in registers
+  const int c = t >> 3, ln = t & 7;                      // column c, rows ln + 8 u
+
+  // ---- S = Q R, reflector j (H_j = I - tau_j v v', v_j = 1, as LAPACK's dlarfg) in column
+  // j of H, formed by column j's lanes as soon as its last update is done
+  double x[R], hv[R];  // hv: reflector c
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int i = ln + 8 * u;
+    x[u] = i < k && c < k ? P.S[i + c * P.lds] : 0.0;
+    hv[u] = 0.0;
+  }
+  auto reflector = [&]() {
+    double a = 0.0, s2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int i = ln + 8 * u;
+      a = i == c ? x[u] : a;
+      s2 = i > c ? __builtin_fma(x[u], x[u], s2) : s2;
     }
-    __syncthreads();
-    const double tj = s_hv[1];
-    if (c < k) {
-      if (c > j && tj != 0.0) {
-        double w = 0.0;
-        for (int i = j + ln; i < k; i += gq) w = __builtin_fma(H[i + j * k], A[i + c * lda], w);
-        w = group_sum_rt(w, gq) * tj;
-        for (int i = j + ln; i < k; i += gq) A[i + c * lda] = __builtin_fma(-w, H[i + j * k], A[i + c * lda]);
-      } else if (c == j) {
-        for (int i = j + ln; i < k; i += gq) A[i + c * lda] = i == j ? s_hv[0] : 0.0;
+    a = group_sum8(a);
+    s2 = group_sum8(s2);
+    double beta = a, tj = 0.0, scale = 0.0;
+    if (s2 > 0.0) {
+      beta = -copysign(sqrt(__builtin_fma(a, a, s2)), a);
+      tj = (beta - a) / beta;
+      scale = 1.0 / (a - beta);
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int i = ln + 8 * u;
+      hv[u] = i == c ? 1.0 : i > c ? x[u] * scale : 0.0;
+      H[i + c * LD] = hv[u];
+      x[u] = i == c ? beta : i > c ? 0.0 : x[u];
+    }
+    if (ln == 0) tau[c] = tj;
+  };
+  if (c == 0) reflector();
+  if (t < 3) s_rot[t] = 0;
+  __syncthreads();
+  for (int j = 0; j < k - 1; ++j) {
+    if (c > j && c < k) {
+      const double tj = tau[j];
+      if (tj != 0.0) {
+        double h[R], w = 0.0;
+#pragma unroll
+        for (int u = 0; u < R; ++u) h[u] = H[ln + 8 * u + j * LD];
+#pragma unroll
+        for (int u = 0; u < R; ++u) w = __builtin_fma(h[u], x[u], w);
+        w = group_sum8(w) * tj;
+#pragma unroll
+        for (int u = 0; u < R; ++u) x[u] = __builtin_fma(-w, h[u], x[u]);
       }
+      if (c == j + 1) reflector();
     }
     __syncthreads();
   }
-  // A <- R' (each pair below/above the diagonal handled by one thread)
-  for (int e = t; e < k * k; e += nt) {
-    const int i = e % k, jj = e / k;
-    if (i > jj) {
-      A[i + jj * lda] = A[jj + i * lda];
-      A[jj + i * lda] = 0.0;
-    }
+  // A = R', V = I; what is past k stays zero (V: the identity) under the rotations
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int i = ln + 8 * u;
+    A[c + i * LD] = x[u];
+    Vm[i + c * LV] = i == c ? 1.0 : 0.0;
+    if constexpr (R > 12) P.work[N * N + t + 64 * R * u] = hv[u];
   }
   __syncthreads();
-}
 
-// X <- Q X = H_0 H_1 ... H_{k-1} X for the reflectors of jacobi_qr_precondition,
-// X k rows x ncols (ld ldx, ncols <= 128), nt threads
-__device__ void jacobi_apply_q(const double* H, const double* tau, int k, double* X, int ldx, int ncols, int nt) {
-  const int t = threadIdx.x;
-  const int cap = ncols > 64 ? 128 : 64;
-  const int gq = nt / cap;
-  const int c = t / gq, ln = t % gq;
-  for (int j = k - 1; j >= 0; --j) {
-    const double tj = tau[j];
-    if (tj != 0.0 && c < ncols) {
-      double w = 0.0;
-      for (int i = j + ln; i < k; i += gq) w = __builtin_fma(H[i + j * k], X[i + c * ldx], w);
-      w = group_sum_rt(w, gq) * tj;
-      for (int i = j + ln; i < k; i += gq) X[i + c * ldx] = __builtin_fma(-w, H[i + j * k], X[i + c * ldx]);
+  // ---- the sweeps
+  const bool vhalf = t >= 32 * R;
+  const int pair = (vhalf ? t - 32 * R : t) >> 3;
+  const bool act = pair < ke / 2;
+  int pa = pair, pb = pair == 0 ? 1 : ke - pair;
+  if (pair) pa = 1 + pair;
+  if (pa > ke - 1) pa = 1;
+  auto next_pair = [&]() {  // columns 1 .. ke - 1 move round
+    if (pair) pa = pa == ke - 1 ? 1 : pa + 1;
+    pb = pb == ke - 1 ? 1 : pb + 1;
+  };
+  auto rotate_v = [&](int b) {
+    const double2 r = cs[b * (N / 2) + pair];
+    if (act && r.y != 0.0) {
+      double u[R], w[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        u[q] = Vm[ln + 8 * q + pa * LV];
+        w[q] = Vm[ln + 8 * q + pb * LV];
+      }
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        Vm[ln + 8 * q + pa * LV] = r.x * u[q] - r.y * w[q];
+        Vm[ln + 8 * q + pb * LV] = r.y * u[q] + r.x * w[q];
+      }
     }
-    __syncthreads();
-  }
-}
-
-constexpr int kJacobiWaveLda = 33;  // odd column stride against bank conflicts
-
-// The same Jacobi sweeps for k <= 32 in one wavefront: G lanes per column pair,
-// rows ln, ln + G, ... of the pair in each lane, the group sums through DPP,
-// no workgroup barriers (LDS operations of one wavefront complete in order).
-template <int G>
-__device__ void jacobi_wave_body(const SvdArgs P, double* __restrict__ A, double* __restrict__ Vm,
-                                 double* __restrict__ sig, double* __restrict__ Hq, double* __restrict__ tq) {
-  constexpr int R = (128 / (G * G)) > 0 ? 128 / (G * G) : 1;  // rows per lane: ke <= 128 / G
-  constexpr int LDA = kJacobiWaveLda;
-  // rows i = ln + G j of every lane stay below 32 unless G = 64 (ke = 2)
-  constexpr bool kGuard = G * R > 32;
-  const int k = P.k;
-  const int ke = (k + 1) & ~1;
-  const int t = threadIdx.x;
-  // the whole arrays: rows and columns past k (A) and ke (V) hold zeros, which
-  // the rotations keep, so the row loops below need no bounds
-  for (int e = t; e < LDA * 32; e += 64) {
-    const int i = e % LDA, j = e / LDA;
-    A[e] = (i < k && j < k) ? P.S[i + j * P.lds] : 0.0;
-    Vm[e] = (i == j && i < ke) ? 1.0 : 0.0;
-  }
-  __syncthreads();
-  jacobi_qr_precondition(A, LDA, k, Hq, tq, 64);  // A <- R' of S = Q R
-  const int npairs = ke / 2;
-  const int pair = t / G, ln = t % G;
+    next_pair();
+  };
+  int buf = 0;
   for (int sweep = 0; sweep < 60; ++sweep) {
     int rot = 0;
+    if (t == 0) s_rot[(sweep + 1) % 3] = 0;
     for (int round = 0; round < ke - 1; ++round) {
-      int pa = 0, pb = 0;
-      const bool act = pair < npairs;
-      if (pair == 0) {
-        pa = 0;
-        pb = 1 + (round % (ke - 1));
-      } else if (act) {
-        pa = 1 + ((round + pair) % (ke - 1));
-        pb = 1 + ((round - pair + (ke - 1)) % (ke - 1));
-      }
-      double x[R], y[R], u[R], w[R];
-      double al = 0.0, be = 0.0, ga = 0.0;
-      // the pair's rows of A and of V, all loaded up front (one LDS wait)
+      if (!vhalf) {
+        if (act) {
+          double y[R], al = 0.0, be = 0.0, ga = 0.0;
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
-        const int i = ln + G * j;
-        const bool ok = !kGuard || i < ke;  // inactive groups read column 0 and never rotate
-        x[j] = ok ? A[i + pa * LDA] : 0.0;
-        y[j] = ok ? A[i + pb * LDA] : 0.0;
-        u[j] = ok ? Vm[i + pa * LDA] : 0.0;
-        w[j] = ok ? Vm[i + pb * LDA] : 0.0;
-      }
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        al = __builtin_fma(x[j], x[j], al);
-        be = __builtin_fma(y[j], y[j], be);
-        ga = __builtin_fma(x[j], y[j], ga);
-      }
-      al = group_sum<G>(al);
-      be = group_sum<G>(be);
-      ga = group_sum<G>(ga);
-      // rotate unless |ga| <= 4 eps sqrt(al be); tan of the angle
-      // t = sign(d) 2ga / (|d| + sqrt(d^2 + 4ga^2)), d = be - al (|t| <= 1),
-      // through refined hardware reciprocals (column norms are normal numbers)
-      if (act && ga * ga > 16.0 * kEps * kEps * al * be) {
-        const double d = be - al;
-        const double g2 = 2.0 * ga;
-        const double q = __builtin_fma(d, d, g2 * g2);
-        const double den = fabs(d) + q * rsqrt_nr(q);
-        double tt = g2 * rcp_nr(den);
-        if (d < 0.0) tt = -tt;
-        const double c = rsqrt_nr(__builtin_fma(tt, tt, 1.0));
-        const double sn = c * tt;
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-          const int i = ln + G * j;
-          if (!kGuard || i < ke) {
-            A[i + pa * LDA] = c * x[j] - sn * y[j];
-            A[i + pb * LDA] = sn * x[j] + c * y[j];
-            Vm[i + pa * LDA] = c * u[j] - sn * w[j];
-            Vm[i + pb * LDA] = sn * u[j] + c * w[j];
+          for (int q = 0; q < R; ++q) {
+            x[q] = A[ln + 8 * q + pa * LD];
+            y[q] = A[ln + 8 * q + pb * LD];
           }
+#pragma unroll
+          for (int q = 0; q < R; ++q) {
+            al = __builtin_fma(x[q], x[q], al);
+            be = __builtin_fma(y[q], y[q], be);
+            ga = __builtin_fma(x[q], y[q], ga);
+          }
+          al = group_sum8(al);
+          be = group_sum8(be);
+          ga = group_sum8(ga);
+          // rotate unless |ga| <= 4 eps sqrt(al be); tan of the angle
+          // t = sign(d) 2ga / (|d| + sqrt(d^2 + 4ga^2)), d = be - al (|t| <= 1),
+          // through refined hardware reciprocals (column norms are normal numbers)
+          double2 r{1.0, 0.0};
+          if (ga * ga > 16.0 * kEps * kEps * al * be) {
+            const double d = be - al;
+            const double g2 = 2.0 * ga;
+            const double q2 = __builtin_fma(d, d, g2 * g2);
+            const double den = fabs(d) + q2 * rsqrt_nr(q2);
+            double tt = g2 * rcp_nr(den);
+            if (d < 0.0) tt = -tt;
+            r.x = rsqrt_nr(__builtin_fma(tt, tt, 1.0));
+            r.y = r.x * tt;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+              A[ln + 8 * q + pa * LD] = r.x * x[q] - r.y * y[q];
+              A[ln + 8 * q + pb * LD] = r.y * x[q] + r.x * y[q];
+            }
+            rot = 1;
+          }
+          if (ln == 0) cs[buf * (N / 2) + pair] = r;
+          next_pair();
         }
-        rot = 1;
+        if (rot && round == ke - 2) s_rot[sweep % 3] = 1;
+      } else if (sweep + round > 0) {
+        rotate_v(buf ^ 1);
       }
-      __builtin_amdgcn_wave_barrier();
-    }
-    if (!__any(rot)) break;
-  }
-  __syncthreads();
-  jacobi_apply_q(Hq, tq, k, Vm, LDA, ke, 64);  // Vm <- Q J
-  jacobi_finish(P, A, LDA, Vm, LDA, sig, 64, true);
-}
-
-
-// The workgroup form (k <= 128, blockDim.x threads): gsz lanes per column pair,
-// a workgroup barrier per round.  A (k x ke) in LDS at an odd stride; V in
-// LDS when it fits, else in P.work.
-__device__ void jacobi_svd_body(const SvdArgs P, double* lds) {
-  const int k = P.k;
-  const int ke = (k + 1) & ~1;
-  const int nt = blockDim.x, t = threadIdx.x;
-  const int lda = k | 1;
-  const int ldv = P.work ? ke : (ke | 1);
-  double* A = lds;                      // k rows x ke columns, ld lda
-  double* sig = A + (size_t)lda * ke;   // ke
-  double* Vm = P.work ? P.work : sig + ke;  // ke x ke, ld ldv
-  // the QR preconditioner's reflectors (k x k) and tau (k): after V, in LDS or
-  // in the global work buffer
-  double* Hq = Vm + (size_t)ldv * ke;
-  double* tq = Hq + (size_t)k * k;
-  for (int e = t; e < ke * k; e += nt) {
-    const int i = e % k, j = e / k;
-    A[i + j * lda] = (j < k) ? P.S[i + j * P.lds] : 0.0;
-  }
-  for (int e = t; e < ke * ke; e += nt) {
-    const int i = e % ke, j = e / ke;
-    Vm[i + j * ldv] = (i == j) ? 1.0 : 0.0;
-  }
-  __syncthreads();
-  jacobi_qr_precondition(A, lda, k, Hq, tq, nt);  // A <- R' of S = Q R
-  const int npairs = ke / 2;
-  int gsz = 1;
-  while (gsz * 2 * npairs <= nt && gsz < 64) gsz *= 2;
-  __shared__ int s_rot;
-  for (int sweep = 0; sweep < 60; ++sweep) {
-    if (t == 0) s_rot = 0;
-    __syncthreads();
-    for (int round = 0; round < ke - 1; ++round) {
-      const int pair = t / gsz, ln = t % gsz;
-      int pa = -1, pb = -1;
-      if (pair < npairs) {
-        if (pair == 0) {
-          pa = 0;
-          pb = 1 + (round % (ke - 1));
-        } else {
-          pa = 1 + ((round + pair) % (ke - 1));
-          pb = 1 + ((round - pair + (ke - 1)) % (ke - 1));
-        }
-      }
-      double al = 0.0, be = 0.0, ga = 0.0;
-      if (pa >= 0) {
-        for (int i = ln; i < k; i += gsz) {
-          const double x = A[i + pa * lda], y = A[i + pb * lda];
-          al = __builtin_fma(x, x, al);
-          be = __builtin_fma(y, y, be);
-          ga = __builtin_fma(x, y, ga);
-        }
-      }
-      al = group_sum_rt(al, gsz);
-      be = group_sum_rt(be, gsz);
-      ga = group_sum_rt(ga, gsz);
-      // rotate unless |ga| <= 4 eps sqrt(al be) (as in the wavefront form)
-      if (pa >= 0 && ga * ga > 16.0 * kEps * kEps * al * be) {
-        const double d = be - al;
-        const double g2 = 2.0 * ga;
-        const double q = __builtin_fma(d, d, g2 * g2);
-        const double den = fabs(d) + q * rsqrt_nr(q);
-        double tt = g2 * rcp_nr(den);
-        if (d < 0.0) tt = -tt;
-        const double c = rsqrt_nr(__builtin_fma(tt, tt, 1.0));
-        const double sn = c * tt;
-        for (int i = ln; i < k; i += gsz) {
-          const double x = A[i + pa * lda], y = A[i + pb * lda];
-          A[i + pa * lda] = c * x - sn * y;
-          A[i + pb * lda] = sn * x + c * y;
-        }
-        for (int i = ln; i < ke; i += gsz) {
-          const double x = Vm[i + pa * ldv], y = Vm[i + pb * ldv];
-          Vm[i + pa * ldv] = c * x - sn * y;
-          Vm[i + pb * ldv] = sn * x + c * y;
-        }
-        if (ln == 0) s_rot = 1;
-      }
+      buf ^= 1;
       __syncthreads();
     }
-    const int any = s_rot;
-    __syncthreads();
-    if (!any) break;
+    if (!s_rot[sweep % 3]) break;
   }
-  jacobi_apply_q(Hq, tq, k, Vm, ldv, ke, nt);  // Vm <- Q J
-  jacobi_finish(P, A, lda, Vm, ldv, sig, nt, true);
+  if (vhalf) rotate_v(buf ^ 1);  // the last round's, if any
+  __syncthreads();
+
+  // ---- column c: the norm, V <- Q J, its place in descending order
+  double s2 = 0.0;
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    x[u] = A[ln + 8 * u + c * LD];
+    s2 = __builtin_fma(x[u], x[u], s2);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    if constexpr (R > 12) hv[u] = P.work[N * N + t + 64 * R * u];
+    H[ln + 8 * u + c * LD] = hv[u];
+  }
+  __syncthreads();
+  double v[R], h[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    v[u] = Vm[ln + 8 * u + c * LV];
+    h[u] = H[ln + 8 * u + (k - 1) * LD];
+  }
+  for (int j = k - 1; j >= 0; --j) {
+    double g[R], w = 0.0;
+    const int jn = j > 0 ? j - 1 : 0;
+#pragma unroll
+    for (int u = 0; u < R; ++u) g[u] = H[ln + 8 * u + jn * LD];
+#pragma unroll
+    for (int u = 0; u < R; ++u) w = __builtin_fma(h[u], v[u], w);
+    w = group_sum8(w) * tau[j];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      v[u] = __builtin_fma(-w, h[u], v[u]);
+      h[u] = g[u];
+    }
+  }
+  const double sg = sqrt(group_sum8(s2));
+  if (ln == 0) sig[c] = sg;
+  __syncthreads();
+  double before = 0.0;
+  for (int l = ln; l < k; l += 8) before += (sig[l] > sg) || (sig[l] == sg && l < c) ? 1.0 : 0.0;
+  const int pos = (int)group_sum8(before);
+  if (c < k) {
+    const double inv = sg > 0.0 ? 1.0 / sg : 0.0;
+    if (ln == 0) {
+      P.sigma[pos] = sg;
+      sorted[pos] = sg;
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int i = ln + 8 * u;
+      if (i < k) {
+        P.V[i + pos * k] = x[u] * inv;
+        P.U[i + pos * k] = v[u];
+      }
+    }
+  }
+  __syncthreads();
+  // lane j: the tail sum from the smallest value up to sigma_j; the rank is one more than
+  // the last j >= 1 whose tail is above tol
+  if (t < 64) {
+    int rho = 1;
+    for (int j0 = 0; j0 < k; j0 += 64) {
+      const int j = j0 + t;
+      double tail = 0.0;
+      for (int l = k - 1; l >= 1; --l) {
+        const double q = sorted[l];
+        if (l >= j) tail = tail + q * q;
+      }
+      const unsigned long long above = __ballot(j >= 1 && j < k && !(sqrt(tail) <= P.tol));
+      if (above) rho = j0 + 64 - __clzll((long long)above);
+    }
+    if (rho > P.rmax) rho = (int)P.rmax;
+    if (rho < 1) rho = 1;
+    if (t == 0) *P.r_out = rho;
+  }
+}
+
+template <bool kBig>
+__device__ void jacobi_dispatch(const SvdArgs P, double* lds) {
+  if constexpr (kBig) {
+    if (P.k <= 80) jacobi_body<10>(P, lds);
+    else if (P.k <= 96) jacobi_body<12>(P, lds);
+    else jacobi_body<16>(P, lds);
+  } else {
+    if (P.k <= 16) jacobi_body<2>(P, lds);
+    else if (P.k <= 32) jacobi_body<4>(P, lds);
+    else if (P.k <= 48) jacobi_body<6>(P, lds);
+    else jacobi_body<8>(P, lds);
+  }
 }
 
 __global__ __launch_bounds__(kThreads) void k_small_abt(const double* __restrict__ A, const double* __restrict__ B,
@@ -2327,106 +2275,51 @@ hipError_t launch_bug_adj_post(BugAdjSmall* A, int r, hipStream_t st) {
   return hipGetLastError();
 }
 
-// workgroup 0 decomposes P0, workgroup 1 (if launched) P1
-__global__ __launch_bounds__(1024) void k_jacobi_svd(SvdArgs P0, SvdArgs P1) {
+// workgroup 0 decomposes P0, workgroup 1 (if launched) P1; kBig: 64 < k <= 128
+template <bool kBig>
+__global__ __launch_bounds__(kBig ? 1024 : 512) void k_jacobi_svd(SvdArgs P0, SvdArgs P1) {
   extern __shared__ double lds[];
-  jacobi_svd_body(blockIdx.x == 0 ? P0 : P1, lds);
-}
-
-__device__ void jacobi_wave_dispatch(const SvdArgs P);
-
-// one wavefront per decomposition, k <= 32 (workgroup b decomposes P_b)
-__global__ __launch_bounds__(64) void k_jacobi_wave(SvdArgs P0, SvdArgs P1) {
-  jacobi_wave_dispatch(blockIdx.x == 0 ? P0 : P1);
+  jacobi_dispatch<kBig>(blockIdx.x == 0 ? P0 : P1, lds);
 }
 
 // the batched forms: one record holds the one or two decompositions of a launch
 struct SvdPair {
   SvdArgs P0, P1;
 };
-__global__ __launch_bounds__(1024) void k_jacobi_svd_batch(const unsigned char* __restrict__ tab,
-                                                           const int* __restrict__ start, int count) {
+template <bool kBig>
+__global__ __launch_bounds__(kBig ? 1024 : 512) void k_jacobi_svd_batch(const unsigned char* __restrict__ tab,
+                                                                        const int* __restrict__ start, int count) {
   extern __shared__ double lds[];
   const int i = batch_member(start, count, blockIdx.x);
   const SvdPair& S = *reinterpret_cast<const SvdPair*>(tab + (size_t)start[count + 1 + i] * kRecArgBytes);
-  jacobi_svd_body(blockIdx.x - start[i] == 0 ? S.P0 : S.P1, lds);
-}
-__global__ __launch_bounds__(64) void k_jacobi_wave_batch(const unsigned char* __restrict__ tab,
-                                                          const int* __restrict__ start, int count) {
-  const int i = batch_member(start, count, blockIdx.x);
-  const SvdPair& S = *reinterpret_cast<const SvdPair*>(tab + (size_t)start[count + 1 + i] * kRecArgBytes);
-  jacobi_wave_dispatch(blockIdx.x - start[i] == 0 ? S.P0 : S.P1);
+  jacobi_dispatch<kBig>(blockIdx.x - start[i] == 0 ? S.P0 : S.P1, lds);
 }
 
-__device__ void jacobi_wave_dispatch(const SvdArgs P) {
-  // one set of LDS arrays for every variant (25.7 KB: several decompositions per CU)
-  __shared__ double A[kJacobiWaveLda * 32];
-  __shared__ double Vm[kJacobiWaveLda * 32];
-  __shared__ double sig[32];
-  __shared__ double Hq[32 * 32];  // the QR preconditioner's reflectors
-  __shared__ double tq[32];
-  const int np = ((P.k + 1) & ~1) / 2;
-  if (np > 8)
-    jacobi_wave_body<4>(P, A, Vm, sig, Hq, tq);
-  else if (np > 4)
-    jacobi_wave_body<8>(P, A, Vm, sig, Hq, tq);
-  else if (np > 2)
-    jacobi_wave_body<16>(P, A, Vm, sig, Hq, tq);
-  else if (np > 1)
-    jacobi_wave_body<32>(P, A, Vm, sig, Hq, tq);
-  else
-    jacobi_wave_body<64>(P, A, Vm, sig, Hq, tq);
+static int jacobi_rows(int k) {
+  return k <= 16 ? 2 : k <= 32 ? 4 : k <= 48 ? 6 : k <= 64 ? 8 : k <= 80 ? 10 : k <= 96 ? 12 : 16;
 }
 
-// LDS doubles of one decomposition; clears P.work when the right factor fits in LDS
-static hipError_t jacobi_plan(SvdArgs& P, size_t* lds) {
-  if (P.k < 1 || P.k > kMaxAug) return hipErrorInvalidValue;
-  const int ke = (P.k + 1) & ~1;
-  *lds = sizeof(double) * ((size_t)(P.k | 1) * ke + ke);  // A and sigma
-  if (P.k <= 64) {
-    // V, the QR preconditioner's reflectors and tau in LDS as well
-    *lds += sizeof(double) * ((size_t)(ke | 1) * ke + (size_t)P.k * P.k + P.k);
-    P.work = nullptr;
-  } else if (!P.work) {
-    return hipErrorInvalidValue;  // V, reflectors and tau in the global work buffer (kSvdWorkDoubles)
-  }
-  return hipSuccess;
-}
-
-// threads of the workgroup form: 8 or more lanes per column pair up to 1024
-static int jacobi_threads(int k) { return k <= 64 ? 512 : 1024; }
-
-hipError_t launch_jacobi_svd(SvdArgs P, hipStream_t st) {
-  size_t lds;
-  hipError_t e = jacobi_plan(P, &lds);
-  if (e != hipSuccess) return e;
-  const SvdPair S{P, P};
-  if (P.k <= 32) {
-    if (!record_launch(KID_JACOBI_WAVE, 0, 1, 64, 0, S))
-      hipLaunchKernelGGL(k_jacobi_wave, dim3(1), dim3(64), 0, st, P, P);
-  } else if (!record_launch(KID_JACOBI_WG, 0, 1, (unsigned)jacobi_threads(P.k), lds, S)) {
-    hipLaunchKernelGGL(k_jacobi_svd, dim3(1), dim3(jacobi_threads(P.k)), lds, st, P, P);
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_jacobi_svd2(SvdArgs P0, SvdArgs P1, hipStream_t st) {
-  size_t l0, l1;
-  hipError_t e = jacobi_plan(P0, &l0);
-  if (e == hipSuccess) e = jacobi_plan(P1, &l1);
-  if (e != hipSuccess) return e;
+static hipError_t launch_jacobi(const SvdArgs& P0, const SvdArgs& P1, unsigned count, hipStream_t st) {
+  const int k = std::max(P0.k, P1.k), R = jacobi_rows(k);
+  const bool big = k > 64;
+  for (const SvdArgs* P : {&P0, &P1})
+    if (P->k < 1 || P->k > kMaxAug || (big && !P->work)) return hipErrorInvalidValue;
+  // R = 12 takes the most: 160 KB to the last 240 bytes
+  const size_t lds = sizeof(double) * (k > 96 && std::min(P0.k, P1.k) > 96 ? jacobi_lds_doubles(16)
+                                       : k > 96                           ? jacobi_lds_doubles(12)
+                                                                          : jacobi_lds_doubles(R));
+  // a batch merges all members up to k = 64 into one launch of 512 threads, of which the
+  // smaller ones' spare waves leave at once: a launch for every size one after
+  // the other would add their times up
   const SvdPair S{P0, P1};
-  if (P0.k <= 32 && P1.k <= 32) {
-    if (!record_launch(KID_JACOBI_WAVE, 0, 2, 64, 0, S))
-      hipLaunchKernelGGL(k_jacobi_wave, dim3(2), dim3(64), 0, st, P0, P1);
-  } else {
-    const unsigned th = (unsigned)jacobi_threads(std::max(P0.k, P1.k));
-    const size_t lds = l0 > l1 ? l0 : l1;
-    if (!record_launch(KID_JACOBI_WG, 0, 2, th, lds, S))
-      hipLaunchKernelGGL(k_jacobi_svd, dim3(2), dim3(th), lds, st, P0, P1);
+  if (!record_launch(KID_JACOBI, big, count, big ? 1024 : 512, lds, S)) {
+    if (big) hipLaunchKernelGGL(k_jacobi_svd<true>, dim3(count), dim3(64 * R), lds, st, P0, P1);
+    else hipLaunchKernelGGL(k_jacobi_svd<false>, dim3(count), dim3(64 * R), lds, st, P0, P1);
   }
   return hipGetLastError();
 }
+hipError_t launch_jacobi_svd(SvdArgs P, hipStream_t st) { return launch_jacobi(P, P, 1, st); }
+hipError_t launch_jacobi_svd2(SvdArgs P0, SvdArgs P1, hipStream_t st) { return launch_jacobi(P0, P1, 2, st); }
 
 // ----------------------------------------------------------------------------
 // orthonormal completion of dropped CholeskyQR columns (see CompleteArgs)
@@ -2658,8 +2551,10 @@ hipError_t launch_rowops_batched(int kid, int variant, const void* tab, const in
       else if (variant == 32) hipLaunchKernelGGL(k_epilogue_batch<32>, g, b, lds, st, t, start, count);
       else hipLaunchKernelGGL(k_epilogue_batch<64>, g, b, lds, st, t, start, count);
       break;
-    case KID_JACOBI_WAVE: hipLaunchKernelGGL(k_jacobi_wave_batch, g, b, lds, st, t, start, count); break;
-    case KID_JACOBI_WG: hipLaunchKernelGGL(k_jacobi_svd_batch, g, b, lds, st, t, start, count); break;
+    case KID_JACOBI:
+      if (variant) hipLaunchKernelGGL(k_jacobi_svd_batch<true>, g, b, lds, st, t, start, count);
+      else hipLaunchKernelGGL(k_jacobi_svd_batch<false>, g, b, lds, st, t, start, count);
+      break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
