@@ -355,12 +355,13 @@ struct PassArgs {
 };
 
 // Choose splits/chunk for a pass whose output has `out_rows` rows and whose
-// reduction runs over `red_len`; returns the partial buffer element count.
+// reduction runs over `red_len`; returns the partial buffer element count.  coarse: fewer
+// splits, for the smallest partial buffer.
 int64_t plan_pass(int mode, bool transposed, int64_t out_rows, int64_t red_len, int rb, int* splits,
-                  int64_t* chunk);
+                  int64_t* chunk, bool coarse = false);
 // The same with a given reduction chunk (rounded up to the 256-row quantum).
 int64_t plan_pass_chunk(int64_t out_rows, int64_t red_len, int rb, int64_t chunk_in, int* splits, int64_t* chunk);
-// The chunks the autotuner times: those for about 128 .. 3072 workgroups, distinct.
+// The chunks the autotuner times: the default, those for about 128 .. 3072 workgroups; distinct.
 int pass_chunk_candidates(int mode, bool transposed, int64_t out_rows, int64_t red_len, int rb, int64_t* chunks,
                           int cap);
 hipError_t launch_passN(int mode, const PassArgs& a, hipStream_t st);

@@ -66,14 +66,14 @@ int rb_for(int mode, int64_t cols) {
 
 // Scratch bytes a call of this shape needs (the packed operand, then the partials).
 static size_t noalloc_need(int mode, bool transposed, int64_t n, int64_t m, int rb, size_t* pk_bytes, int* splits,
-                           int64_t* chunk) {
+                           int64_t* chunk, bool coarse) {
   const int64_t krows = transposed ? n : m;  // rows of B
   const int64_t kpad = (krows + 63) / 64 * 64;
   size_t pk = 0;
   if (mode == PASS_F64) pk = sizeof(double) * (size_t)kpad * rb;
   else if (mode == PASS_F32) pk = sizeof(float) * (size_t)kpad * rb;
   else pk = 2 * 2 * (size_t)kpad * rb;  // hi and lo panels
-  const int64_t parts = plan_pass(mode, transposed, transposed ? m : n, transposed ? n : m, rb, splits, chunk);
+  const int64_t parts = plan_pass(mode, transposed, transposed ? m : n, transposed ? n : m, rb, splits, chunk, coarse);
   *pk_bytes = align256(pk);
   return *pk_bytes + align256((size_t)parts * (mode == PASS_F64 ? 8 : 4));
 }
@@ -99,7 +99,16 @@ extern "C" int lri_product_noalloc(int which, int dtype, int precision, int64_t 
   size_t pk_bytes = 0;
   int splits = 0;
   int64_t chunk = 0;
-  const size_t need = noalloc_need(mode, tr, n, m, rb, &pk_bytes, &splits, &chunk);
+  // what the scratch has to hold is the coarse plan; the finer default is taken where it fits too
+  const size_t need = noalloc_need(mode, tr, n, m, rb, &pk_bytes, &splits, &chunk, true);
+  if (need <= kNoAllocScratchBytes) {
+    int s;
+    int64_t ch;
+    if (noalloc_need(mode, tr, n, m, rb, &pk_bytes, &s, &ch, false) <= kNoAllocScratchBytes) {
+      splits = s;
+      chunk = ch;
+    }
+  }
   if (need > kNoAllocScratchBytes)
     return fail(LRI_EINVAL, "n = " + std::to_string(n) + ", m = " + std::to_string(m) + ", r = " + std::to_string(r) +
                                 " needs " + std::to_string(need) + " bytes of scratch, above LRI_NOALLOC_SCRATCH_BYTES = " +

@@ -23,6 +23,7 @@
 //  f32 32x32x2:   A lane l -> A[l%32][l/32]; B lane l -> B[l/32][l%32]; D as bf16.
 // Only the pairing of A and B along k matters for a product, so the kernels
 // assign k indices to (lane, element) freely as long as A and B agree.
+#include <algorithm>
 #include "lri_common.h"
 #include "lri_kernels.h"
 #include "../../include/lri.h"
@@ -1154,14 +1155,14 @@ static int wg_span(int mode, bool transposed, int rb) {
 
 constexpr int64_t kChunkQuantum = 256;  // 4 waves x the largest per-wave iteration (64 rows)
 
-// The reduction chunk for about `target` workgroups, with at least 1024 of the
+// The reduction chunk for about `target` workgroups, with at least `least` of the
 // reduction range per split.
 static int64_t chunk_for_target(int mode, bool transposed, int64_t out_rows, int64_t red_len, int rb,
-                                int64_t target) {
+                                int64_t target, int64_t least) {
   const int span = wg_span(mode, transposed, rb);
   const int64_t tiles = (out_rows + span - 1) / span;
   int64_t want = (target + tiles - 1) / tiles;
-  const int64_t maxs = (red_len + 1023) / 1024;
+  const int64_t maxs = (red_len + least - 1) / least;
   if (want > maxs) want = maxs;
   if (want < 1) want = 1;
   const int64_t ch = (red_len + want - 1) / want;
@@ -1177,21 +1178,33 @@ int64_t plan_pass_chunk(int64_t out_rows, int64_t red_len, int rb, int64_t ch, i
   return s * rb * out_rows;
 }
 
-// the default: ~512 workgroups (2048 waves); ~768 for the BF16 pass N at rb <= 32,
-// whose 64-row workgroups run four waves per SIMD (at n = m = 16384: 3 splits, 170
-// us against 196 us for 2)
+// The default.  Full: ~512 workgroups (2048 waves) with 1024 of the reduction each; ~768 for
+// the BF16 pass N at rb <= 32, whose 64-row workgroups run four waves per SIMD (at n = m =
+// 16384: 3 splits, 170 us against 196 us for 2).  Where that leaves fewer than 512
+// workgroups, a wave's chain of loads is what bounds the pass, and splits down to 256 of
+// the reduction cost less than they shorten it, though the partial results grow
+// (FP64 2000 x 1500: N 41 -> 18 us with 6 splits for 2, T 66 -> 21 us with 8; FP32 10007 x
+// 4099: 135 -> 108, 145 -> 107; BF16 8192 x 3000: 26 -> 21, 28 -> 26).  The FP64 passes
+// hold fewer bytes in flight per wave and gain up to 1536 workgroups (6144 x 8192 at r = 48:
+// N 277 -> 202 us with 8 splits for 3, T 236 -> 227 with 6 for 2).
+// coarse: without the finer splits (the smallest partial results).
 int64_t plan_pass(int mode, bool transposed, int64_t out_rows, int64_t red_len, int rb, int* splits,
-                  int64_t* chunk) {
+                  int64_t* chunk, bool coarse) {
   const int64_t target = (mode == PASS_BF16X3 && !transposed && rb <= 32) ? 768 : 512;
-  return plan_pass_chunk(out_rows, red_len, rb, chunk_for_target(mode, transposed, out_rows, red_len, rb, target),
-                         splits, chunk);
+  int64_t ch = chunk_for_target(mode, transposed, out_rows, red_len, rb, target, 1024);
+  if (!coarse) {
+    ch = std::min(ch, chunk_for_target(mode, transposed, out_rows, red_len, rb, 512, 256));
+    if (mode == PASS_F64) ch = std::min(ch, chunk_for_target(mode, transposed, out_rows, red_len, rb, 1536, 512));
+  }
+  return plan_pass_chunk(out_rows, red_len, rb, ch, splits, chunk);
 }
 
 int pass_chunk_candidates(int mode, bool transposed, int64_t out_rows, int64_t red_len, int rb, int64_t* chunks,
                           int cap) {
-  int k = 0;
+  int k = 0, s;
+  if (cap > 0) plan_pass(mode, transposed, out_rows, red_len, rb, &s, &chunks[k++]);
   for (int64_t target : {128, 192, 256, 384, 512, 640, 768, 1024, 1280, 1536, 2048, 3072}) {
-    const int64_t ch = chunk_for_target(mode, transposed, out_rows, red_len, rb, target);
+    const int64_t ch = chunk_for_target(mode, transposed, out_rows, red_len, rb, target, 256);
     bool dup = false;
     for (int i = 0; i < k; ++i) dup = dup || chunks[i] == ch;
     if (!dup && k < cap) chunks[k++] = ch;
