@@ -243,10 +243,10 @@ struct SvdArgs {
   int* r_out = nullptr;
   double tol = 0.0;
   int64_t rmax = 0;
-  double* work = nullptr;  // global scratch of kSvdWorkDoubles for k > 64 (V, the QR preconditioner)
+  double* work = nullptr;  // global scratch of kSvdWorkDoubles, given for k > 64, used above 96
 };
-// the global Jacobi work of one decomposition with k > 64: V (ke x ke), the
-// preconditioner's reflectors (k x k) and tau (k)
+// the global Jacobi work of one decomposition with k > 64: V and the preconditioner's
+// reflectors (128 x 128 each)
 constexpr int kSvdWorkDoubles = 2 * kMaxAug * kMaxAug + kMaxAug;
 hipError_t launch_jacobi_svd(SvdArgs P, hipStream_t st);
 
